@@ -792,6 +792,7 @@ bp_status bp_dispatch_matmul_q1_0(bp_model* m, const void* weights, const void* 
     a.a_qs_offset = a_qs;
     a.out_offset = out_off;
     a.accumulate = accumulate ? 1u : 0u;
+    a.cu_count = static_cast<uint32_t>(m->cu_count);
     return hip_check(m, bp::launch_matmul_q1_0_q8_0(a, m->stream), "matmul_q1_0_q8_0 launch");
 }
 

@@ -187,6 +187,7 @@ struct MatmulArgs {
     uint32_t w_d_offset, w_qs_offset, a_d_offset, a_qs_offset;   // bytes
     uint32_t out_offset;      // f16 elements
     uint32_t accumulate;
+    uint32_t cu_count;
 };
 struct TopKArgs {
     const uint16_t* logits;   // f16 activation buffer

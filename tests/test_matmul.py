@@ -215,6 +215,37 @@ def test_matmul_bit_exact(cuda, m, n, k, acc):
     assert bad.size == 0, f"{bad.size} outputs differ, first at {bad[:8]}"
 
 
+# Every kernel choice at its edges (3 workgroups per CU of 256): the split kernel
+# (8 blocks a chunk: 1, 7, 8, 9 and 17 blocks), 16 tokens a workgroup (4 blocks a
+# stage), 32 tokens with 4 and with 2 blocks a stage; ragged rows and tokens, n not
+# a multiple of 4, offsets that are multiples of 4 only.
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,acc,shift", [
+    (1, 1, 128, 0, 0), (17, 33, 7 * 128, 1, 4), (16, 16, 8 * 128, 0, 8), (33, 50, 9 * 128, 1, 0), (15, 70, 17 * 128, 0, 4),
+    (193, 1000, 5 * 128, 1, 4), (200, 1001, 3 * 128, 0, 0), (250, 3001, 4 * 128, 0, 0), (250, 3004, 6 * 128, 1, 4),
+    (209, 5003, 6 * 128, 1, 4), (223, 7001, 3 * 128, 0, 4), (200, 8200, 2 * 128, 1, 0), (225, 6404, 5 * 128, 0, 8)])
+def test_matmul_kernel_choices_bit_exact(cuda, m, n, k, acc, shift):
+    _say(f"[matmul choices] m={m} n={n} k={k} acc={acc} shift={shift}")
+    rng = np.random.default_rng(m + n + k + shift)
+    wbuf, w_d, w_qs = _weights(rng, n, k, pad=256 + shift)
+    d_off, qs_off, size = _q8_layout(m, k)
+    d_off, qs_off, size = d_off + shift, qs_off + shift, size + shift
+    x = (rng.standard_normal(m * k) * np.exp(2 * rng.standard_normal(m * k))).astype(np.float16)
+    q8 = orc.quantize_act_q8_0(orc.QuantParams(k=k, m=m, input_offset=0, d_offset=d_off, qs_offset=qs_off),
+                               _f16(x), np.zeros(size, np.uint8))
+    out_off = 40 + (shift >> 2)
+    y0 = _f16(rng.standard_normal(out_off + m * n + 40))
+    p = orc.MatmulParams(k=k, n=n, m=m, w_d_offset=w_d, w_qs_offset=w_qs, a_d_offset=d_off, a_qs_offset=qs_off,
+                         out_offset=out_off, accumulate=acc)
+    want = orc.matmul_q1_0_q8_0(p, wbuf, q8, y0)
+    w_dv, q_dv, y_dv = _dev(wbuf), _dev(q8), _dev(y0)
+    _model().dispatch_matmul_q1_0(w_dv.data_ptr(), q_dv.data_ptr(), y_dv.data_ptr(), k, n, m, w_d, w_qs, d_off,
+                                  qs_off, out_off, bool(acc))
+    got = _host(y_dv, np.uint16)
+    bad = np.flatnonzero(got != want)
+    assert bad.size == 0, f"{bad.size} outputs differ, first at {bad[:8]}"
+
+
 @pytest.mark.gpu
 def test_quantize_then_matmul_on_device(cuda):
     """The reference's two-dispatch sequence on the device (quantize into the
