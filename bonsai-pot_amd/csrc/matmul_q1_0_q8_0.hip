@@ -38,57 +38,52 @@ namespace {
 typedef int i4v __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------- quantize
-// One thread per 32-element block: 64 bytes in (four 16-byte loads), the
-// block max in registers, 32 quantized bytes + one f32 d out. Per element the
-// operations are the reference's (|x| max, one IEEE divide for d, one for
-// 1/d, rne(x * inv), clamp), so the bytes are identical.
+// Four lanes per 32-element block: 16 bytes in, the block max by two lane
+// exchanges, 8 quantized bytes out (one thread per block read and wrote with a
+// 64-byte stride and left the chip emptier). Per element the operations are the
+// reference's (|x| max, one IEEE divide for d, one for 1/d, rne(x * inv),
+// clamp), so the bytes are identical.
 __global__ __launch_bounds__(256) void quantize_act_q8_0_kernel(QuantArgs a) {
     const uint32_t nb = a.k / 32;
-    const uint32_t blk = blockIdx.x * 256 + threadIdx.x;   // row * nb + b
+    const uint32_t gid = blockIdx.x * 256 + threadIdx.x;
+    const uint32_t blk = gid >> 2, part = gid & 3;   // blk = row * nb + b
     if (blk >= a.m * nb) return;
-    const uint32_t row = blk / nb, b = blk % nb;
-    const uint16_t* src = a.act + a.input_offset + static_cast<uint64_t>(row) * a.k + 32 * b;
-    uint32_t w[16];
+    const uint64_t at = 32 * static_cast<uint64_t>(blk) + 8 * part;   // row * k + 32 b + 8 part
+    const uint16_t* src = a.act + a.input_offset + at;
+    uint32_t w[4];
     if ((reinterpret_cast<uintptr_t>(src) & 15u) == 0) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint4 q = reinterpret_cast<const uint4*>(src)[i];
-            w[4 * i] = q.x; w[4 * i + 1] = q.y; w[4 * i + 2] = q.z; w[4 * i + 3] = q.w;
-        }
+        const uint4 q = *reinterpret_cast<const uint4*>(src);
+        w[0] = q.x; w[1] = q.y; w[2] = q.z; w[3] = q.w;
     } else {   // input_offset not a multiple of 8 elements: element loads
 #pragma unroll
-        for (int i = 0; i < 16; i++) w[i] = static_cast<uint32_t>(src[2 * i]) | (static_cast<uint32_t>(src[2 * i + 1]) << 16);
+        for (int i = 0; i < 4; i++) w[i] = static_cast<uint32_t>(src[2 * i]) | (static_cast<uint32_t>(src[2 * i + 1]) << 16);
     }
-    float v[32];
+    float v[8];
     float amax = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
+    for (int i = 0; i < 4; i++) {
         v[2 * i] = h2f(static_cast<uint16_t>(w[i] & 0xFFFFu));
         v[2 * i + 1] = h2f(static_cast<uint16_t>(w[i] >> 16));
         amax = fmaxf(amax, fmaxf(fabsf(v[2 * i]), fabsf(v[2 * i + 1])));
     }
+    amax = fmaxf(amax, lane_xor<1>(amax));
+    amax = fmaxf(amax, lane_xor<2>(amax));
     const float d = amax / 127.0f;
     const float inv = d > 0.0f ? 1.0f / d : 0.0f;
-    uint32_t out[8];
+    uint32_t out[2] = {0, 0};
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        uint32_t word = 0;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const float r = fminf(fmaxf(rintf(v[4 * i + e] * inv), -127.0f), 127.0f);
-            word |= (static_cast<uint32_t>(static_cast<int32_t>(r)) & 0xFFu) << (8 * e);
-        }
-        out[i] = word;
+    for (int e = 0; e < 8; e++) {
+        const float r = fminf(fmaxf(rintf(v[e] * inv), -127.0f), 127.0f);
+        out[e / 4] |= (static_cast<uint32_t>(static_cast<int32_t>(r)) & 0xFFu) << (8 * (e % 4));
     }
-    uint4* qs = reinterpret_cast<uint4*>(a.out + a.qs_offset + static_cast<uint64_t>(row) * a.k + 32 * b);
-    if ((reinterpret_cast<uintptr_t>(qs) & 15u) == 0) {
-        qs[0] = make_uint4(out[0], out[1], out[2], out[3]);
-        qs[1] = make_uint4(out[4], out[5], out[6], out[7]);
+    uint32_t* qs = reinterpret_cast<uint32_t*>(a.out + a.qs_offset + at);
+    if ((reinterpret_cast<uintptr_t>(qs) & 7u) == 0) {
+        *reinterpret_cast<uint2*>(qs) = make_uint2(out[0], out[1]);
     } else {   // qs_offset a multiple of 4 only
-#pragma unroll
-        for (int i = 0; i < 8; i++) reinterpret_cast<uint32_t*>(qs)[i] = out[i];
+        qs[0] = out[0];
+        qs[1] = out[1];
     }
-    *reinterpret_cast<float*>(a.out + a.d_offset + 4 * static_cast<uint64_t>(blk)) = d;
+    if (part == 0) *reinterpret_cast<float*>(a.out + a.d_offset + 4 * static_cast<uint64_t>(blk)) = d;
 }
 
 // ---------------------------------------------------------------- matmul
@@ -400,7 +395,7 @@ void launch_tiles(const MatmulArgs& a, hipStream_t s) {
 
 hipError_t launch_quantize_act_q8_0(const QuantArgs& a, hipStream_t s) {
     const uint32_t blocks = a.m * (a.k / 32);
-    hipLaunchKernelGGL(quantize_act_q8_0_kernel, dim3((blocks + 255) / 256), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(quantize_act_q8_0_kernel, dim3((blocks + 63) / 64), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
