@@ -27,8 +27,9 @@
 //    (hi + lo, so the weights keep f32-like precision), V bytes transposed
 //    into the B layout with v_perm_b32.
 //  * The row sets of a KV head are merged through LDS (log-sum-exp) into one
-//    partial (o[128], m, l) per query head; with a single split the output is
-//    written directly and the merge pass is skipped.
+//    partial (o[128], m, l) per query head. At the shortest contexts one
+//    workgroup of 8 waves takes a KV head's whole context (the single layout),
+//    adds row `pos` itself in the fused step and stores the output: no merge pass.
 //
 // Merge pass (decode_merge_kernel) — one 64-lane workgroup per (query head,
 // 32-dim chunk): log-sum-exp over the splits (attention_merge.wgsl:85-129),
@@ -41,7 +42,7 @@
 // same bits) and, in the last split's workgroup, the kv_writeback of the new
 // row `pos`; it streams rows [0, pos). The merge pass then adds row `pos`
 // (whose bytes are in the cache by then) and writes the normalized q into
-// act. One decode step is two launches instead of four.
+// act. One decode step is two launches instead of four (one in the single layout).
 #include "bp_kernels.hpp"
 #include "bp_norm_rope.hpp"
 
@@ -59,8 +60,10 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 //  kH = 1: 4 waves, all on one KV head, each streaming every 4th 16-row batch;
 //  kH = 4: 8 waves, wave w on KV head 4 hg + (w & 3) and row set w >> 2, so the
 //          4 heads read the same rows together (512 contiguous bytes per row).
-template <int kH> struct SplitShape {
-    static constexpr int kWaves = kH == 1 ? 4 : 8;
+// kSingle (kH = 1): the whole context in one workgroup of 8 waves per KV head,
+//          which also stores the output: one launch, no partials.
+template <int kH, bool kSingle = false> struct SplitShape {
+    static constexpr int kWaves = kH == 1 && !kSingle ? 4 : 8;
     static constexpr int kThreads = 64 * kWaves;
     static constexpr int kRowSets = kWaves / kH;
     static constexpr int kWgPerCu = 8 / kWaves;   // at 2 waves per SIMD
@@ -112,13 +115,17 @@ __device__ __forceinline__ float sum_slots(float v) {
     return sum_xor32(sum_xor16(v + dpp_f<0x128>(v)));   // row_ror:8 == xor 8 within 16 lanes
 }
 
-template <bool kFused, int kH>
-__global__ __launch_bounds__(SplitShape<kH>::kThreads, SplitShape<kH>::kWgPerCu) void decode_split_kernel(DecodeArgs a) {
-    constexpr int kWaves = SplitShape<kH>::kWaves, kRowSets = SplitShape<kH>::kRowSets;
-    constexpr int kQPerWave = kH * kGroup / kWaves;   // query heads normalized per wave (fused)
+template <bool kFused, int kH, bool kSingle, class Shape = SplitShape<kH, kSingle>>
+__global__ __launch_bounds__(Shape::kThreads, Shape::kWgPerCu) void decode_split_kernel(DecodeArgs a) {
+    constexpr int kWaves = Shape::kWaves, kRowSets = Shape::kRowSets;
+    constexpr int kQWaves = kWaves < kH * kGroup ? kWaves : kH * kGroup;   // waves that normalize q (fused)
+    constexpr int kQPerWave = kH * kGroup / kQWaves;                       // query heads each of them
+    constexpr int kWbWave = kSingle ? 4 : 0;                               // first of the 2 kH writeback waves
     __shared__ __attribute__((aligned(16))) float o_red[kWaves][kGroup][kHeadDim + 4];   // per-wave O
     __shared__ float ml_sh[kWaves][kGroup][2];
     __shared__ __attribute__((aligned(16))) uint16_t qn_sh[kH][kGroup][kHeadDim];
+    __shared__ float new_sh[kSingle ? 2 : 1][kSingle ? kHeadDim : 1];   // row `pos` of K and V as the cache holds it
+    __shared__ float s_new_sh[kGroup];                                  // its score per query head, log2 units
 
     const int t = threadIdx.x;
     const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);   // uniform: scalar registers
@@ -193,10 +200,11 @@ __global__ __launch_bounds__(SplitShape<kH>::kThreads, SplitShape<kH>::kWgPerCu)
     uint16_t qxr[kQPerWave][2] = {}, w0r = 0, w1r = 0, x0r = 0, x1r = 0, kw0r = 0, kw1r = 0;
     uint32_t csr = 0;
     Q16 qraw[4];   // q of head hq, dims 32 lg + 8 i .. +8
-    // Fused step: wave w normalizes the workgroup's query heads kQPerWave w ..,
-    // and waves w < 2 kH write row `pos` of KV head kH hg + (w % kH): K for
-    // w < kH, V otherwise.
-    const uint32_t qh0 = hg * kH * kGroup + kQPerWave * wave;
+    // Fused step: wave w < kQWaves normalizes the workgroup's query heads
+    // kQPerWave w .., and waves w >= kWbWave, w' = w - kWbWave < 2 kH write row
+    // `pos` of KV head kH hg + (w' % kH): K for w' < kH, V otherwise.
+    const int qw = wave % kQWaves, wb = wave - kWbWave;
+    const uint32_t qh0 = hg * kH * kGroup + kQPerWave * qw;
     const uint32_t g_wb = hg * kH + wave % kH;
     if constexpr (kFused) {
         const uint16_t* qr = a.q + static_cast<uint64_t>(qh0) * kHeadDim;
@@ -208,7 +216,7 @@ __global__ __launch_bounds__(SplitShape<kH>::kThreads, SplitShape<kH>::kWgPerCu)
         w0r = a.w_norms[a.w_q_off + lane];
         w1r = a.w_norms[a.w_q_off + lane + 64];
         csr = *reinterpret_cast<const uint32_t*>(cs);
-        const uint16_t* src = (wave < kH ? a.k_cur : a.v_cur) + g_wb * kHeadDim;   // writeback input
+        const uint16_t* src = (wb < kH ? a.k_cur : a.v_cur) + g_wb * kHeadDim;   // writeback input
         x0r = src[lane];
         x1r = src[lane + 64];
         kw0r = a.w_norms[a.w_k_off + lane];
@@ -233,36 +241,52 @@ __global__ __launch_bounds__(SplitShape<kH>::kThreads, SplitShape<kH>::kWgPerCu)
         float x0 = h2f(x0r), x1 = h2f(x1r);
         const float kw0 = h2f(kw0r), kw1 = h2f(kw1r);
         // q_norm_rope (q_norm_rope_fused.wgsl:38-96), into LDS.
-        uint16_t* qn = &qn_sh[0][0][0] + kQPerWave * wave * kHeadDim;
-        uint16_t* qg = a.q_norm + static_cast<uint64_t>(qh0) * kHeadDim;
+        // A single workgroup reads the raw q of its own heads only, so it stores
+        // the normalized q in act itself; else the merge pass does.
+        uint16_t* qn = &qn_sh[0][0][0] + kQPerWave * qw * kHeadDim;
+        uint16_t* qg = (kSingle ? a.q_act : a.q_norm) + static_cast<uint64_t>(qh0) * kHeadDim;
+        if (kQWaves == kWaves || wave < kQWaves) {
 #pragma unroll
-        for (int i = 0; i < kQPerWave; i++) {
-            float o0, o1;
-            norm_rope_pair(qx[i][0], qx[i][1], w0, w1, c0, s0, a.eps, o0, o1);
-            qn[i * kHeadDim + lane] = f2h(o0);
-            qn[i * kHeadDim + lane + 64] = f2h(o1);
-            if (split == 0) {
-                qg[i * kHeadDim + lane] = f2h(o0);
-                qg[i * kHeadDim + lane + 64] = f2h(o1);
+            for (int i = 0; i < kQPerWave; i++) {
+                float o0, o1;
+                norm_rope_pair(qx[i][0], qx[i][1], w0, w1, c0, s0, a.eps, o0, o1);
+                qn[i * kHeadDim + lane] = f2h(o0);
+                qn[i * kHeadDim + lane + 64] = f2h(o1);
+                if (split == 0) {
+                    qg[i * kHeadDim + lane] = f2h(o0);
+                    qg[i * kHeadDim + lane + 64] = f2h(o1);
+                }
             }
         }
-        if (split == a.n_splits - 1 && wave < 2 * kH) {
+        if (split == a.n_splits - 1 && wb >= 0 && wb < 2 * kH) {
             // kv_writeback of row `pos` for KV head g_wb (kv_writeback_fused.wgsl):
             // K (norm + RoPE + Q8_0) or V (Q8_0).
             const uint64_t d_idx = static_cast<uint64_t>(a.pos) * nb_row + g_wb * (kHeadDim / kBlock);
             const uint64_t qs_idx = static_cast<uint64_t>(a.pos) * kv_dim + g_wb * kHeadDim;
-            if (wave < kH) {
+            float n0, n1;
+            if (wb < kH) {
                 norm_rope_pair(x0, x1, kw0, kw1, c0, s0, a.eps, x0, x1);
                 quantize_store_pair(x0, x1, lane, const_cast<float*>(a.k.d) + d_idx,
-                                    const_cast<int8_t*>(a.k.qs) + qs_idx);
+                                    const_cast<int8_t*>(a.k.qs) + qs_idx, n0, n1);
             } else {
                 quantize_store_pair(x0, x1, lane, const_cast<float*>(a.v.d) + d_idx,
-                                    const_cast<int8_t*>(a.v.qs) + qs_idx);
+                                    const_cast<int8_t*>(a.v.qs) + qs_idx, n0, n1);
+            }
+            if constexpr (kSingle) {
+                new_sh[wb][lane] = n0;
+                new_sh[wb][lane + 64] = n1;
             }
         }
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < 4; i++) qraw[i] = *reinterpret_cast<const Q16*>(&qn_sh[hw][hq][32 * lg + 8 * i]);
+        if constexpr (kSingle) {
+            if (wave < kGroup) {   // score of row `pos` for head `wave`
+                const float s = wave_sum(h2f(qn_sh[0][wave][lane]) * new_sh[0][lane] +
+                                         h2f(qn_sh[0][wave][lane + 64]) * new_sh[0][lane + 64]);
+                if (lane == 0) s_new_sh[wave] = s * c2;
+            }
+        }
     }
     // ---- B operand of q.k: q of head hq on block bq's k slots, zero elsewhere;
     // and the bias 1152 * sum(q over block bq) of the exact-f16 K trick. -----------
@@ -441,10 +465,10 @@ __global__ __launch_bounds__(SplitShape<kH>::kThreads, SplitShape<kH>::kWgPerCu)
 
     // ---- merge the row sets: thread t -> query head t / (128 / kE) of the
     // workgroup's 4 kH (KV head fw, its head fh), dims kE (t % (128 / kE)) .. ----
-    constexpr int kE = kH * kGroup * kHeadDim / (64 * kWaves);   // 2 or 4 dims per thread
+    constexpr int kE = kH * kGroup * kHeadDim / (64 * kWaves);   // 1 (single), 2 or 4 dims per thread
     constexpr int kTpH = kHeadDim / kE;                           // threads per query head
     const int fq = t / kTpH, fw = fq >> 2, fh = fq & 3, fd = kE * (t % kTpH);
-    float M = -INFINITY;
+    float M = kSingle && kFused ? s_new_sh[fh] : -INFINITY;
 #pragma unroll
     for (int r = 0; r < kRowSets; r++) M = fmaxf(M, ml_sh[fw + kH * r][fh][0]);
     float L = 0.0f;
@@ -459,20 +483,22 @@ __global__ __launch_bounds__(SplitShape<kH>::kThreads, SplitShape<kH>::kWgPerCu)
         for (int k = 0; k < kE; k++) o[k] = __builtin_fmaf(e, o_red[w][fh][fd + k], o[k]);
     }
     const uint32_t qhd = (hg * kH + fw) * kGroup + fh;
-    if (!kFused && a.n_splits == 1) {
-        const float inv_l = 1.0f / L;
-#pragma unroll
-        for (int k = 0; k < kE; k += 2)
-            *reinterpret_cast<uint32_t*>(a.out + static_cast<uint64_t>(qhd) * kHeadDim + fd + k) =
-                static_cast<uint32_t>(f2h(o[k] * inv_l)) | (static_cast<uint32_t>(f2h(o[k + 1] * inv_l)) << 16);
+    if constexpr (kSingle) {
+        if constexpr (kFused) {   // row `pos`
+            const float w_new = __builtin_amdgcn_exp2f(s_new_sh[fh] - M);
+            L += w_new;
+            o[0] = __builtin_fmaf(w_new, new_sh[1][fd], o[0]);
+        }
+        a.out[static_cast<uint64_t>(qhd) * kHeadDim + fd] = f2h(o[0] * (1.0f / L));
         return;
-    }
-    float* part = part_o(a.partials, qhd, a.n_splits, split);
+    } else {
+        float* part = part_o(a.partials, qhd, a.n_splits, split);
 #pragma unroll
-    for (int k = 0; k < kE; k += 2) *reinterpret_cast<float2*>(part + fd + k) = make_float2(o[k], o[k + 1]);
-    if (t % kTpH == 0)
-        *reinterpret_cast<float2*>(part_ml(a.partials, a.kv_dim / kHeadDim * kGroup, qhd, a.n_splits, split)) =
-            make_float2(M, L);
+        for (int k = 0; k + 1 < kE; k += 2) *reinterpret_cast<float2*>(part + fd + k) = make_float2(o[k], o[k + 1]);
+        if (t % kTpH == 0)
+            *reinterpret_cast<float2*>(part_ml(a.partials, a.kv_dim / kHeadDim * kGroup, qhd, a.n_splits, split)) =
+                make_float2(M, L);
+    }
 }
 
 // One wave per (query head, 32-dim chunk); kLoads = 8 (up to 64 splits) or
@@ -617,6 +643,18 @@ void decode_plan(uint32_t n_rows, uint32_t n_kv_head, int cu_count, uint32_t min
     uint32_t want = (target + groups - 1) / groups;
     if (want < 1) want = 1;
     if (want > kMaxSplits) want = kMaxSplits;
+    // Up to three batches per wave the whole context of a KV head goes to one
+    // workgroup (n_splits = 1: the single layout), because the merge pass costs a
+    // launch: us per fused step at 100 / 200 / 300 / 500 rows 5.3 / 5.8 / 6.5 /
+    // 8.9, as split + merge 8.0 / 7.7 / 7.9 / 7.9 (calls in a row; graph replays
+    // at 300 and 500 6.6 and 9.0 against 6.7 and 7.1). A batch costs a wave about
+    // 1 us: two waves a SIMD issue an instruction every three cycles each.
+    if (h == 1 && n_rows <= 3 * min_split_rows) {
+        *split_len = (n_rows + 15) / 16 * 16;
+        *n_splits = 1;
+        *heads_per_wg = 1;
+        return;
+    }
     uint32_t len = (n_rows + want - 1) / want;
     if (len < min_split_rows) len = min_split_rows;
     len = (len + batch_rows - 1) / batch_rows * batch_rows;
@@ -628,14 +666,20 @@ void decode_plan(uint32_t n_rows, uint32_t n_kv_head, int cu_count, uint32_t min
 uint32_t decode_max_splits() { return kMaxSplits; }
 uint32_t decode_partial_stride() { return kPartStride; }
 
+// One split of one KV head per workgroup: the single layout, no merge pass.
+static bool decode_single(const DecodeArgs& a) { return a.n_splits == 1 && a.heads_per_wg == 1; }
+
 template <bool kFused>
 static void launch_split(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s) {
     const uint32_t z = (a.n_splits + 7) / 8;
-    if (a.heads_per_wg == 4)
-        hipLaunchKernelGGL((decode_split_kernel<kFused, 4>), dim3(8, n_kv_head / 4, z),
+    if (decode_single(a))
+        hipLaunchKernelGGL((decode_split_kernel<kFused, 1, true>), dim3(1, n_kv_head, 1),
+                           dim3(SplitShape<1, true>::kThreads), 0, s, a);
+    else if (a.heads_per_wg == 4)
+        hipLaunchKernelGGL((decode_split_kernel<kFused, 4, false>), dim3(8, n_kv_head / 4, z),
                            dim3(SplitShape<4>::kThreads), 0, s, a);
     else
-        hipLaunchKernelGGL((decode_split_kernel<kFused, 1>), dim3(8, n_kv_head, z),
+        hipLaunchKernelGGL((decode_split_kernel<kFused, 1, false>), dim3(8, n_kv_head, z),
                            dim3(SplitShape<1>::kThreads), 0, s, a);
 }
 
@@ -661,14 +705,15 @@ static void launch_merge(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s)
 
 hipError_t launch_decode(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s) {
     launch_split<false>(a, n_kv_head, s);
-    if (a.n_splits > 1)
+    if (!decode_single(a))
         launch_merge<false>(a, n_kv_head, s);
     return hipGetLastError();
 }
 
 hipError_t launch_decode_step(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s) {
     launch_split<true>(a, n_kv_head, s);
-    launch_merge<true>(a, n_kv_head, s);
+    if (!decode_single(a))
+        launch_merge<true>(a, n_kv_head, s);
     return hipGetLastError();
 }
 

@@ -37,8 +37,9 @@ __device__ __forceinline__ void norm_rope_pair(float x0, float x1, float w0, flo
 
 // Q8_0-quantize the pair and store it; lanes 0-31 own blocks 0 and 2, lanes
 // 32-63 blocks 1 and 3 (kv_writeback_fused.wgsl:118-200).
-__device__ __forceinline__ void quantize_store_pair(float x0, float x1, int lane, float* d_row,
-                                                    int8_t* qs_row) {
+// deq0 / deq1 receive the pair as the cache now holds it, d * q in f32.
+__device__ __forceinline__ void quantize_store_pair(float x0, float x1, int lane, float* d_row, int8_t* qs_row,
+                                                    float& deq0, float& deq1) {
     float a0 = fabsf(x0), a1 = fabsf(x1);
     a0 = fmaxf(a0, lane_xor<1>(a0)); a1 = fmaxf(a1, lane_xor<1>(a1));
     a0 = fmaxf(a0, lane_xor<2>(a0)); a1 = fmaxf(a1, lane_xor<2>(a1));
@@ -50,6 +51,8 @@ __device__ __forceinline__ void quantize_store_pair(float x0, float x1, int lane
     float i1 = d1 > 0.0f ? 1.0f / d1 : 0.0f;
     int q0 = static_cast<int>(fminf(fmaxf(rintf(x0 * i0), -127.0f), 127.0f));
     int q1 = static_cast<int>(fminf(fmaxf(rintf(x1 * i1), -127.0f), 127.0f));
+    deq0 = d0 * static_cast<float>(q0);
+    deq1 = d1 * static_cast<float>(q1);
     // Gather 4 consecutive lanes' bytes into one little-endian word.
     uint32_t p = (static_cast<uint32_t>(q0) & 0xffu) | ((static_cast<uint32_t>(q1) & 0xffu) << 8);
     const uint32_t p0 = quad_bcast<0>(p), p1 = quad_bcast<1>(p), p2 = quad_bcast<2>(p), p3 = quad_bcast<3>(p);

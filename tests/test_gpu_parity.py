@@ -388,3 +388,28 @@ def test_prefill_key_split(cuda, monkeypatch, m, pos_base, ksplit):
     dev.attention(0, pos_base, is_prefill=True)
     want = sc.oracle_attention(0, pos_base, is_prefill=True)
     assert_attn_close(dev.out_f32(), want, f"prefill key split m={m} pos_base={pos_base} ksplit={ksplit}")
+
+
+# The single layout (one workgroup per KV head, up to 3 x 128 rows) at the edges of
+# its batches and where the split layout takes over; rows of a second model without
+# it (BP_DECODE_MIN_SPLIT_ROWS 32: splits of 64 rows) agree within the same bar.
+@pytest.mark.parametrize("pos", [0, 1, 15, 16, 17, 127, 128, 129, 255, 383, 384, 385])
+def test_decode_single_layout(cuda, monkeypatch, pos):
+    _say(f"[decode single] pos={pos}")
+    cfg = layout.Config(n_layer=2)
+    for min_rows in ("128", "32"):
+        monkeypatch.setenv("BP_DECODE_MIN_SPLIT_ROWS", min_rows)
+        sc = Scenario(cfg, max_seq=pos + 8, m_tokens=1, seed=700 + pos, w_std=0.2)
+        _prefill_cache(sc, 1, pos, seed=800 + pos)
+        dev = DeviceScenario(sc, upload_kv=True)
+        dev.decode_step(1, pos)
+        sc.oracle_q_norm_rope(pos)
+        sc.oracle_writeback(1, pos)
+        k, v = dev.kv_host()
+        assert np.array_equal(k, sc.kv_k) and np.array_equal(v, sc.kv_v), "cache bytes differ"
+        q = slice(sc.q_off, sc.q_off + cfg.q_dim)
+        assert np.array_equal(dev.act_host()[q], sc.act[q]), "normalized q differs"
+        _, want = sc.oracle_decode(1, pos)
+        assert_attn_close(dev.out_f32(1)[0], want, f"decode step pos={pos}")
+        dev.decode(1, pos)
+        assert_attn_close(dev.out_f32(1)[0], want, f"decode pos={pos}")
