@@ -24,6 +24,8 @@
 // per two elements, from pre-shifted copies of the inverted qs word whose
 // bytes are 0x3C | (sign << 7); then one v_pk_fma_f16 adds +-x to the lane's
 // two accumulators. (fma(+-1, x, c) rounds once, exactly as c + (+-x) does.)
+#include <algorithm>
+
 #include "bp_device.hpp"
 #include "bp_kernels.hpp"
 
@@ -136,8 +138,7 @@ __global__ __launch_bounds__(kMvMaxThreads) void matvec_q1_0_kernel(MatvecArgs a
     const uint32_t rows = a.rows_per_wg;
     float* terms = reinterpret_cast<float*>(x_sh + nb * kBlockHalves);   // [rows][nb]
 
-    // This workgroup's rows lie in one range (ranges are multiples of 16 rows
-    // and rows_per_wg divides 16).
+    // This workgroup's rows lie in one range (rows_per_wg divides all but the last).
     const uint32_t row0 = blockIdx.x * rows;
     uint32_t d_off = a.range[0].d_offset, qs_off = a.range[0].qs_offset, out_off = a.range[0].output_offset;
     uint32_t rbase = row0;                       // first row of the workgroup within its range
@@ -261,25 +262,37 @@ hipError_t launch_matvec_q1_0(const MatvecArgs& args, int mode, hipStream_t s) {
     MatvecArgs a = args;
     const uint32_t nb = a.k / kQ1Block, tcols = (nb + 3) / 4;
     // Rows per workgroup and waves: one tile per wave while the whole grid
-    // fits on the GPU at once (8192 waves); else two per wave. The silu matvec
-    // stages an expensive x, so it shares each staging among 16 rows. The
-    // normed sum of squares is defined over 256 threads (4 waves at least).
-    auto plan = [&](uint32_t rows, uint32_t tiles_per_wave) {
+    // fits on the GPU at once (8192 waves). The silu matvec stages an expensive
+    // x, so it shares each staging among 16 rows. The normed sum of squares is
+    // defined over 256 threads (4 waves at least).
+    // Larger grids stage x once for 32 rows (64 from 2048 workgroups of those on)
+    // and use 8 waves, a multiple of the CU's 4 SIMDs: with one tile row's 5 waves
+    // (k = 2560) the first SIMD of a CU got two waves of every workgroup. us before
+    // (16 rows, two tiles per wave) and now: 19456 x 2560 7.2, 7.05; 24576 x 4096
+    // 11.0, 9.9; 32000 x 2048 8.0, 7.7; 151936 x 2560 37, 28.6 (32 rows: 29.2).
+    // Several ranges: rows have to divide them (16 always does); and x and the
+    // terms have to fit 64 KB of LDS.
+    auto plan = [&](uint32_t rows) {
         a.rows_per_wg = rows;
-        const uint32_t tiles = rows / 8 * tcols;
-        uint32_t w = (tiles + tiles_per_wave - 1) / tiles_per_wave;
-        w = w > 16 ? 16 : w;
+        const uint32_t w = std::min(rows / 8 * tcols, 16u);
         return mode == 2 && w < 4 ? 4u : w;
     };
+    auto lds_bytes = [&](uint32_t rows) { return static_cast<size_t>(nb) * kBlockHalves * 2 + static_cast<size_t>(rows) * nb * 4; };
     uint32_t waves;
     if (mode == 1) {
-        waves = plan(16, 1);
+        waves = plan(16);
     } else {
-        waves = plan(8, 1);
-        if (((a.n_total + 7) / 8) * waves > 8192) waves = plan(16, 2);
+        waves = plan(8);
+        if (((a.n_total + 7) / 8) * waves > 8192) {
+            uint32_t rows = a.n_total >= 64 * 2048 ? 64 : 32;
+            const bool one_range = a.range[0].n == a.n_total;
+            while (rows > 16 && ((!one_range && (a.range[0].n % rows || a.range[1].n % rows)) || lds_bytes(rows) > 65536)) rows /= 2;
+            a.rows_per_wg = rows;
+            waves = rows == 16 ? 4 : 8;
+        }
     }
     const uint32_t n_wg = (a.n_total + a.rows_per_wg - 1) / a.rows_per_wg;
-    const size_t lds = static_cast<size_t>(nb) * kBlockHalves * 2 + static_cast<size_t>(a.rows_per_wg) * nb * 4;
+    const size_t lds = lds_bytes(a.rows_per_wg);
     const dim3 block(64 * waves);
     if (mode == 0)
         hipLaunchKernelGGL(matvec_q1_0_kernel<0>, dim3(n_wg), block, lds, s, a);

@@ -444,3 +444,48 @@ def test_matvec_rejects_bad_shapes(cuda, monkeypatch):
     with pytest.raises(PotError):
         m.dispatch_matvec_q1_0_fused_normed(w.data_ptr(), a.data_ptr(), a.data_ptr(), 256, 0, 0,
                                             [(0, 0, 24, 0)])
+
+
+# The f16-order kernel's larger grids (32 or 64 rows a workgroup, 8 waves; 16 rows
+# where a range is no multiple of 32), with rows past the last whole workgroup.
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k,acc", [(65600, 128, 0), (65601, 512, 1), (131072, 128, 0), (131072 + 33, 256, 1)])
+def test_matvec_large_grids(cuda, monkeypatch, n, k, acc):
+    _say(f"[matvec large] n={n} k={k} acc={acc}")
+    rng = np.random.default_rng(n + k)
+    buf, [(d_off, qs_off)] = _weights(rng, [(n, k)])
+    act = _f16(rng.standard_normal(k + n + 64))
+    p = orc.MatvecParams(k=k, n=n, d_offset=d_off, qs_offset=qs_off, input_offset=0, output_offset=k + 24,
+                         accumulate=acc)
+    want = orc.matvec_q1_0(p, buf, act)
+    w_d, a_d = _dev(buf), _dev(act)
+    _model(monkeypatch, "f16").dispatch_matvec_q1_0(w_d.data_ptr(), a_d.data_ptr(), k, n, d_off, qs_off, 0, k + 24, bool(acc))
+    bad = np.flatnonzero(_host(a_d) != want)
+    assert bad.size == 0, f"{bad.size} f16 outputs differ, first at {bad[:8]}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [(32768, 32800), (32784, 32784), (16, 32768, 32784), (64, 131072), (0, 65568)])
+def test_matvec_fused_normed_large_grids(cuda, monkeypatch, sizes):
+    """Each range must be the product one range alone gives (small grids, bit-exact above)."""
+    import torch
+    k = 256
+    _say(f"[matvec normed large] sizes={sizes}")
+    rng = np.random.default_rng(sum(sizes))
+    buf, offs = _weights(rng, [(n, k) for n in sizes])
+    total = sum(sizes)
+    act = _f16(rng.standard_normal(k + total + 64))
+    norms = _f16(1 + 0.1 * rng.standard_normal(k))
+    m = _model(monkeypatch, "f16")
+    w_d, n_d = _dev(buf), _dev(norms)
+    at = np.concatenate([[0], np.cumsum(sizes)[:-1]]) + k + 8
+    ranges = [(d, q, n, int(o)) for (d, q), n, o in zip(offs, sizes, at)]
+    got_d, want_d = _dev(act), _dev(act)
+    m.dispatch_matvec_q1_0_fused_normed(w_d.data_ptr(), got_d.data_ptr(), n_d.data_ptr(), k, 0, 0, ranges)
+    for d, q, n, o in ranges:
+        for lo in range(0, n, 8192):   # pieces that run one tile per wave
+            c = min(8192, n - lo)
+            m.dispatch_matvec_q1_0_fused_normed(w_d.data_ptr(), want_d.data_ptr(), n_d.data_ptr(), k, 0, 0,
+                                                [(d + 2 * lo * (k // 128), q + 16 * lo * (k // 128), c, o + lo)])
+    torch.cuda.synchronize()
+    assert torch.equal(got_d, want_d)
