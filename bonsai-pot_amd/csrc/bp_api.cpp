@@ -44,7 +44,6 @@ struct bp_model {
     uint64_t partials_floats;
     uint16_t* kv16;       // prefill: image of one layer's K and V (prefill_image_bytes)
     uint16_t* q_norm;     // decode-step scratch: normalized q, [n_head][128] f16
-    uint32_t* readback;   // pinned host words that bp_topk_readback's copy kernel writes
     uint32_t decode_min_split_rows;
     uint32_t decode_wide_min_rows;
     uint32_t prefill_hpw;   // 0 = by grid size; 2 = prefill32_kernel, 1 = the one-head 16x16 kernels
@@ -313,8 +312,7 @@ bp_status bp_model_create(const bp_config* cfg, uint32_t max_seq, int device, bp
         hipMalloc(&m->rope_cs, rope_elems * 2) != hipSuccess ||
         hipMalloc(&m->partials, m->partials_floats * 4) != hipSuccess ||
         hipMalloc(&m->q_norm, static_cast<size_t>(cfg->n_head) * cfg->head_dim * 2) != hipSuccess ||
-        hipMalloc(&m->kv16, bp::prefill_image_bytes(cfg->n_kv_head, max_seq)) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void**>(&m->readback), 4 * bp::kReadbackWords, hipHostMallocDefault) != hipSuccess) {
+        hipMalloc(&m->kv16, bp::prefill_image_bytes(cfg->n_kv_head, max_seq)) != hipSuccess) {
         (void)hipGetLastError();
         return bail(fail(BP_ERR_OUT_OF_MEMORY, "hipMalloc failed for KV cache of %llu bytes x2",
                          static_cast<unsigned long long>(m->kv_bytes)));
@@ -340,7 +338,6 @@ void bp_model_destroy(bp_model* m) {
         if (m->partials) (void)hipFree(m->partials);
         if (m->kv16) (void)hipFree(m->kv16);
         if (m->q_norm) (void)hipFree(m->q_norm);
-        if (m->readback) (void)hipHostFree(m->readback);
     }
     (void)hipGetLastError();
     delete m;
@@ -823,17 +820,18 @@ bp_status bp_topk_readback(bp_model* m, const void* result, uint32_t out_off, ui
     if (st != BP_OK) return st;
     if (!result || (k && (!values || !indices))) return fail(BP_ERR_INVALID_ARG, "result/values/indices is NULL");
     if (k > 32) return fail(BP_ERR_INVALID_ARG, "topk readback k = %u exceeds 32", k);
-    // One copy kernel into pinned memory and one wait (a synchronous copy of the
-    // values and one of the indices took 40 us together with their waits).
+    // Values and indices lie together: one copy on the stream and one wait.
+    uint32_t words[2 * bp::kTopKMax];
     if (k != 0) {
         const uint32_t* src = static_cast<const uint32_t*>(result) + out_off;
-        if ((st = hip_check(m, bp::launch_copy_words(src, m->readback, 2 * k, m->stream), "topk readback copy")) != BP_OK)
+        if ((st = hip_check(m, hipMemcpyAsync(words, src, 8ull * k, hipMemcpyDeviceToHost, m->stream),
+                            "topk readback copy")) != BP_OK)
             return st;
     }
     if ((st = hip_check(m, hipStreamSynchronize(m->stream), "topk readback sync")) != BP_OK) return st;
     if (k == 0) return BP_OK;
-    std::memcpy(values, m->readback, 4ull * k);
-    std::memcpy(indices, m->readback + k, 4ull * k);
+    std::memcpy(values, words, 4ull * k);
+    std::memcpy(indices, words + k, 4ull * k);
     return BP_OK;
 }
 

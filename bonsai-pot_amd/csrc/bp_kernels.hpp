@@ -195,9 +195,7 @@ struct TopKArgs {
     uint32_t n, in_offset, out_offset, k;   // in_offset: f16 elements (rounded down to even)
 };
 hipError_t launch_topk_reduce(const TopKArgs& a, hipStream_t s);
-// Copies n <= kReadbackWords words to pinned host memory (visible once the stream is waited for).
-constexpr uint32_t kReadbackWords = 64;
-hipError_t launch_copy_words(const uint32_t* src, uint32_t* host, uint32_t n, hipStream_t s);
+constexpr uint32_t kTopKMax = 32;
 hipError_t launch_quantize_act_q8_0(const QuantArgs& a, hipStream_t s);
 hipError_t launch_matmul_q1_0_q8_0(const MatmulArgs& a, hipStream_t s);
 

@@ -623,20 +623,10 @@ __global__ __launch_bounds__(kThreads) void topk_kernel(TopKArgs a) {
     }
 }
 
-// One wave: the readback of the result words into pinned host memory.
-__global__ __launch_bounds__(64) void copy_words_kernel(const uint32_t* src, uint32_t* host, uint32_t n) {
-    if (threadIdx.x < n) host[threadIdx.x] = src[threadIdx.x];
-}
-
 }  // namespace
 
 hipError_t launch_topk_reduce(const TopKArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(topk_kernel, dim3(1), dim3(kThreads), 0, s, a);
-    return hipGetLastError();
-}
-
-hipError_t launch_copy_words(const uint32_t* src, uint32_t* host, uint32_t n, hipStream_t s) {
-    hipLaunchKernelGGL(copy_words_kernel, dim3(1), dim3(kReadbackWords), 0, s, src, host, n);
     return hipGetLastError();
 }
 
