@@ -4,16 +4,18 @@
 // attends rows [0, cur) with cur = causal ? pos + m + 1 : pos, f32 softmax,
 // f16 output. Three forms, chosen by the host from the shapes:
 //
-// 1. Image pass + prefill32_kernel (long prompts): kv_dequant_kernel (or the
+// 1. Image pass + prefill32_kernel: kv_dequant_kernel (or the
 //    fused step's prefill_prep_kernel) writes the layer's K and V for rows
 //    [0, cur of the last token) as an f16 image (f16(d * q) per value, plus a
 //    K residual below), per KV head and 64-row chunk laid out as its LDS
 //    image, so that a chunk is one linear copy; prefill32_kernel runs on
 //    v_mfma_f32_32x32x16_f16 with 4 query heads x 32 tokens per role and the
-//    two waves of each SIMD one phase apart (its own comment below).
-// 2. Image pass + prefill_kernel<1, 8> / <1, 4> (shorter prompts): one query
-//    head per wave on v_mfma_f32_16x16x32_f16, two or four workgroups per
-//    (KV head, tile pair), so that small grids still fill the CUs.
+//    two waves of each SIMD one phase apart (its own comment below). Grids
+//    that leave CUs idle take one tile per workgroup instead of two and, on
+//    few tiles, split the keys as well (then prefill_merge_kernel).
+// 2. Image pass + prefill_kernel<1, 4> (few key chunks; <1, 8> when forced):
+//    one query head per wave on v_mfma_f32_16x16x32_f16, four (two) workgroups
+//    per (KV head, tile pair), so that small grids still fill the CUs.
 // 3. prefill_split_kernel + prefill_merge_kernel (few tokens over a long
 //    cache): the keys split over workgroups that read the cache's Q8_0 rows
 //    themselves (no image), partials merged by their log-sum-exp weights.
@@ -910,7 +912,13 @@ __global__ __launch_bounds__(64) void prefill_merge_kernel(PrefillArgs a) {
 //
 //  * Workgroup: 8 waves, one KV head g and a zig-zag pair of 32-token tiles
 //    (light A = p, heavy B = n_tiles - 1 - p), processed one after the other,
-//    so every pair runs about (n_A + n_B) / 2 iterations. Wave w owns query
+//    so every pair runs about (n_A + n_B) / 2 iterations; or one tile, heaviest
+//    first, where pairs would leave half of the CUs idle (the step is bound by
+//    one workgroup's chain of steps then: 777 tokens on 1501 rows 60.7 -> 49.8
+//    us, 512 on 4096 82 -> 67 with the keys split as well). With a key split,
+//    blockIdx.y takes the split's chunks of the tile and the workgroup writes
+//    (O, m, l) to kpart for prefill_merge_kernel; a split past a tile's last
+//    key writes m = -inf. Wave w owns query
 //    head 4 g + (w & 3) for the tile's 32 tokens; "Y" waves (w >= 4) take the
 //    first half of the tile's key chunks, "X" waves (w < 4) the second half,
 //    and the halves are merged through LDS (log-sum-exp) at the end of the
@@ -981,11 +989,14 @@ __global__ __launch_bounds__(512) void prefill32_kernel(PrefillArgs a) {
     float m_run = -INFINITY, l_run = 0.0f;   // l_run: this lane's keys only
     bool have_p = false;
 
-    // Keys [0, kend) the tile attends, its 64-key chunks and the Y / X split.
+    // Keys [0, kend) the tile attends, its 64-key chunks (of this key split, from
+    // chunk c_lo on) and the Y / X split.
+    const uint32_t split = blockIdx.y, c_lo = split * a.split_chunks;   // 0 without a key split
     auto tile_geom = [&](uint32_t tile, uint32_t& kend, uint32_t& n, uint32_t& md) __attribute__((always_inline)) {
         const uint32_t last = min(tile * kPrefillTileTok + kPrefillTileTok, a.m_tokens) - 1;
         kend = a.causal ? a.pos + last + 1 : a.pos;
         n = (kend + kChunk - 1) / kChunk;
+        if (a.n_ksplit > 1) n = min(max(n, c_lo) - c_lo, a.split_chunks);
         md = (n + 1) / 2;
     };
     // Loads of a tile's q into qb (waited for where they are used).
@@ -1042,6 +1053,20 @@ __global__ __launch_bounds__(512) void prefill32_kernel(PrefillArgs a) {
                 w.y = pack2(o[dt][4 * j + 2] * inv_l, o[dt][4 * j + 3] * inv_l);
                 *reinterpret_cast<uint2*>(out + 32 * dt + 8 * j + 4 * g8) = w;
             }
+    };
+
+    // Key split: O (unnormalized), m (log2 units) and l of this split.
+    auto write_partial = [&](float m, float l_tot) __attribute__((always_inline)) {
+        if (!unit_live || my_tok >= a.m_tokens) return;
+        const uint32_t n_head = a.q_stride / kHeadDim;
+        float* pp = a.kpart + ((static_cast<uint64_t>(my_tok) * n_head + head) * a.n_ksplit + split) * kSplitStride;
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                *reinterpret_cast<f32x4*>(pp + 32 * dt + 8 * j + 4 * g8) =
+                    f32x4{o[dt][4 * j], o[dt][4 * j + 1], o[dt][4 * j + 2], o[dt][4 * j + 3]};
+        if (g8 == 0) *reinterpret_cast<float2*>(pp + kHeadDim) = make_float2(m, l_tot);
     };
 
     // ---- copies: 16-byte pieces, 1 KB per wave and instruction -------------
@@ -1229,12 +1254,12 @@ __global__ __launch_bounds__(512) void prefill32_kernel(PrefillArgs a) {
     auto issue_tile = [&](uint32_t tile) __attribute__((always_inline)) {
         uint32_t kend, n, md;
         tile_geom(tile, kend, n, md);
-        const uint32_t ch0 = is_x ? md : 0u, cnt = is_x ? n - md : md;
+        const uint32_t ch0 = c_lo + (is_x ? md : 0u), cnt = is_x ? n - md : md;
         if (cnt > 0) copy_k4(is_x ? k2a : k1a, ch0);
         issue_q(tile);
     };
     auto process = [&]() __attribute__((always_inline)) {
-        const uint32_t ch0 = is_x ? mid : 0u;                // this role's first chunk
+        const uint32_t ch0 = c_lo + (is_x ? mid : 0u);       // this role's first chunk
         const uint32_t cnt = is_x ? n_ch - mid : mid;        // and its chunk count
         uint16_t* const kst0 = is_x ? k2a : k1a;             // this role's stages
         uint16_t* const kst1 = is_x ? k2b : k1b;
@@ -1314,12 +1339,13 @@ __global__ __launch_bounds__(512) void prefill32_kernel(PrefillArgs a) {
             for (int dt = 0; dt < 4; dt++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) o[dt][r] = o[dt][r] * ey + xo[(dt * 16 + r) * 64 + lane] * ex;
-            write_out(l_tot * ey + lx * ex);
+            if (a.n_ksplit > 1) write_partial(mm, l_tot * ey + lx * ex);
+            else write_out(l_tot * ey + lx * ex);
         }
         barrier_lds();   // the merge area is the next tile's stages
     };
 
-    const uint32_t tile_a = pair, tile_b = a.n_tiles - 1 - pair;   // tile_b >= tile_a
+    const uint32_t tile_b = a.n_tiles - 1 - pair, tile_a = a.tiles_per_wg == 1 ? tile_b : pair;   // tile_b >= tile_a
     issue_tile(tile_a);
     enter_tile(tile_a);
     for (uint32_t tile = tile_a;; tile = tile_b) {   // (one code instance for both tiles)
@@ -1634,14 +1660,18 @@ static void launch_prefill_merge(const PrefillArgs& a, uint32_t n_kv_head, hipSt
         hipLaunchKernelGGL(prefill_merge_kernel<32>, grid, dim3(64), 0, s, a);
 }
 
+static bool prefill_one_tile(const PrefillArgs& a) { return a.heads_per_wave == 2 && a.tiles_per_wg == 1; }
+
 static void launch_attention(const PrefillArgs& a, uint32_t n_kv_head, hipStream_t s) {
     const uint32_t n_pairs = (a.n_tiles + 1) / 2;
     if (a.direct) {
         hipLaunchKernelGGL(prefill_split_kernel, dim3(n_kv_head, a.n_ksplit, n_pairs), dim3(512), 0, s, a);
         launch_prefill_merge(a, n_kv_head, s);
-    } else if (a.heads_per_wave == 2)
-        hipLaunchKernelGGL(prefill32_kernel, dim3(n_kv_head, 1, n_pairs), dim3(512), 0, s, a);
-    else if (a.wg_waves == 4)
+    } else if (a.heads_per_wave == 2) {
+        hipLaunchKernelGGL(prefill32_kernel, dim3(n_kv_head, a.n_ksplit, prefill_one_tile(a) ? a.n_tiles : n_pairs),
+                           dim3(512), 0, s, a);
+        if (a.n_ksplit > 1) launch_prefill_merge(a, n_kv_head, s);
+    } else if (a.wg_waves == 4)
         hipLaunchKernelGGL((prefill_kernel<1, 4>), dim3(n_kv_head, 4, n_pairs), dim3(256), 0, s, a);
     else
         hipLaunchKernelGGL((prefill_kernel<1, 8>), dim3(n_kv_head, 2, n_pairs), dim3(512), 0, s, a);
@@ -1650,7 +1680,7 @@ static void launch_attention(const PrefillArgs& a, uint32_t n_kv_head, hipStream
 // HIP's grid limit in y and z.
 constexpr uint64_t kGridYZMax = 65535;
 static uint64_t attention_grid_z(const PrefillArgs& a) {
-    return (a.n_tiles + 1) / 2;
+    return prefill_one_tile(a) ? a.n_tiles : (a.n_tiles + 1) / 2;
 }
 // Preparation pass, grid y: the image's halves (or with no image, the halves
 // holding new rows), then kGroup q parts per half holding new rows.

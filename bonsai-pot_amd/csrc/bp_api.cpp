@@ -527,48 +527,74 @@ static bp_status prefill_args(bp_model* m, void* act, uint32_t q_off, uint32_t o
     a.causal = is_prefill ? 1u : 0u;
     a.n_tiles = (m_tokens + bp::kPrefillTileTok - 1) / bp::kPrefillTileTok;
     {
-        // The one-head 16x16 kernels (two 8-wave workgroups per tile pair and KV
-        // head, each wave 16 tokens of one query head) while that grid still
-        // fits the compute units at one workgroup each, else prefill32_kernel
-        // (one 8-wave workgroup per tile pair and KV head; at 64-1024 tokens it
-        // measured 12.0-32.5 us against 10.1-27.3 us for the 16x16 kernels).
-        // Then 4-wave workgroups (four per tile pair and KV head) while those
-        // fit. BP_PREFILL_HEADS_PER_WAVE and BP_PREFILL_WG_WAVES force a layout.
-        const uint32_t pairs = (a.n_tiles + 1) / 2;
+        const uint32_t pairs = (a.n_tiles + 1) / 2, n_kv = m->cfg.n_kv_head;
         const uint32_t cus = static_cast<uint32_t>(m->cu_count > 0 ? m->cu_count : 256);
-        a.heads_per_wave = m->prefill_hpw != 0 ? m->prefill_hpw : (2 * pairs * m->cfg.n_kv_head <= cus ? 1u : 2u);
-        a.wg_waves = 8;
-        if (a.heads_per_wave == 1)
-            a.wg_waves = m->prefill_waves != 0 ? m->prefill_waves : (4 * pairs * m->cfg.n_kv_head <= cus ? 4u : 8u);
-        // Key split for short chunks over long caches (where the 4-wave
-        // layout would be chosen): split every tile pair's key range over
-        // n_ksplit workgroups (fewer splits when the partials would not fit),
-        // then merge. BP_PREFILL_KSPLIT forces a split count (within the
-        // partials).
+        const uint32_t chunks = static_cast<uint32_t>((rows + 63) / 64);   // the last tile's key chunks
+        const uint64_t cap = m->partials_floats / (static_cast<uint64_t>(m->cfg.n_head) * kPrefillSplitStride);
+        const bool small = 4 * pairs * n_kv <= cus;   // the 4-wave layout of the 16x16 kernels fits the CUs
         a.n_ksplit = 1;
         a.split_chunks = 0;
         a.kpart = m->partials;
         a.direct = 0;
-        const uint32_t chunks = static_cast<uint32_t>((rows + 63) / 64);   // the last tile's key chunks
-        if (a.heads_per_wave == 1 && a.wg_waves == 4 && is_prefill &&
-            (m->prefill_ksplit != 0 || chunks >= 4 * a.n_tiles)) {
-            // prefill_split_kernel for few tiles over a long cache (at least 4
-            // key chunks per tile): one 8-wave workgroup per (KV head, key
-            // split, tile pair) reading the cache rows itself; enough splits
-            // to give every CU a workgroup, at least 2 chunks each.
-            const uint32_t wgs = pairs * m->cfg.n_kv_head;                   // workgroups per split
-            uint32_t ns = m->prefill_ksplit != 0
-                              ? m->prefill_ksplit
-                              : std::min<uint32_t>(std::max<uint32_t>((cus + wgs - 1) / wgs, 1u), chunks / 2);
-            const uint64_t cap = m->partials_floats / (static_cast<uint64_t>(m->cfg.n_head) * kPrefillSplitStride);
+        auto split_keys = [&](uint32_t ns) {
             ns = std::min<uint32_t>(ns, 64);   // prefill_merge_kernel: one split per lane
             while (ns > 1 && static_cast<uint64_t>(m_tokens) * ns > cap) --ns;
             if (ns > 1) {
                 a.n_ksplit = ns;
                 a.split_chunks = (chunks + ns - 1) / ns;
+            }
+            return ns > 1;
+        };
+        // Kernel (us of the fused step below; BP_PREFILL_HEADS_PER_WAVE,
+        // BP_PREFILL_WG_WAVES and BP_PREFILL_KSPLIT force one):
+        //  * prefill_kernel, the one-head 16x16 kernel with 4 waves, for at most 5
+        //    key chunks, and 8 while at most a quarter of the rows lie before the
+        //    chunk (half the scores of its tile pairs are masked): 64 / 256 / 448
+        //    tokens from an empty cache 12.1 / 16.4 / 19.3, prefill32_kernel 14.5 /
+        //    17.0 / 20.5; but 200 on 250 rows 21.6 and 20.1;
+        //  * prefill_split_kernel (reads the cache's own rows, no image) for few
+        //    tiles over a long cache, from 32 chunks per tile on, where writing the
+        //    image costs more than converting in the workgroups (64 tokens on 16384
+        //    rows 54, prefill32_kernel 69; 128 on 8192 52 and 51), and for a single
+        //    tile (16 on 500 / 1000 rows 16.0 / 16.0, prefill32_kernel 20.1 / 20.9);
+        //  * else prefill32_kernel.
+        a.heads_per_wave = m->prefill_hpw != 0 ? m->prefill_hpw : 2u;
+        if (m->prefill_hpw != 2 && is_prefill && small && m->prefill_waves != 8 &&
+            (m->prefill_ksplit != 0 || chunks >= (a.n_tiles == 1 ? 6 : 32 * a.n_tiles))) {
+            // one 8-wave workgroup per (KV head, key split, tile pair): enough splits
+            // to give every CU a workgroup, at least 2 chunks each (a single tile: 1,
+            // up to 16 splits; 16 tokens on 1000 rows: 8 splits 16.9, 16 16.0)
+            const uint32_t wgs = pairs * n_kv;
+            uint32_t most = chunks / 2;
+            if (a.n_tiles == 1) most = std::max(most, std::min(chunks, 16u));
+            if (split_keys(m->prefill_ksplit != 0 ? m->prefill_ksplit : std::min<uint32_t>((cus + wgs - 1) / wgs, most))) {
                 a.direct = 1;
+                a.heads_per_wave = 1;
             }
         }
+        const bool few = chunks <= 5 || (chunks <= 8 && 4 * static_cast<uint64_t>(m_tokens) >= 3 * rows);
+        if (m->prefill_hpw == 0 && !a.direct && small && (few || m->prefill_waves != 0)) a.heads_per_wave = 1;
+        a.wg_waves = 8;
+        if (a.heads_per_wave == 1) a.wg_waves = m->prefill_waves != 0 ? m->prefill_waves : (small ? 4u : 8u);
+        // prefill32_kernel: one tile per workgroup while all tiles fit the CUs (512
+        // tokens on 2048 rows 48.6, as pairs 74.6; 777 on 1501 49.8 and 67.6), or
+        // while the tiles beyond them are so light that two take less than the
+        // heaviest one (1025 tokens from an empty cache 31.1 and 38.0); else zig-zag
+        // pairs (2048: 65.8 and 64.2; 1200 on 3000: 122 and 116).
+        const uint32_t wgs = a.n_tiles * n_kv;
+        a.tiles_per_wg = 2;
+        if (wgs <= cus) {
+            a.tiles_per_wg = 1;
+        } else if (wgs <= 2 * cus && is_prefill) {
+            const uint32_t next = a.n_tiles - 1 - cus / n_kv;   // the heaviest tile beyond the first round
+            a.tiles_per_wg = 2 * ((static_cast<uint64_t>(pos) + 32 * next + 95) / 64) < chunks ? 1 : 2;
+        }
+        // One tile per workgroup on at most half the CUs: split its keys too, at least
+        // 6 chunks and one per 20 tokens each (the partials and the merge grow with
+        // the tokens): 64 tokens on 1000 rows 27.3 -> 24.9, 256 on 4096 71.0 -> 47.0,
+        // 512 on 4096 76.0 -> 67.0; but 512 on 1024 33.9 -> 38.5 when split.
+        if (a.heads_per_wave == 2 && a.tiles_per_wg == 1 && is_prefill && m->prefill_hpw == 0)
+            split_keys(std::min(cus / wgs, chunks / std::max(6u, m_tokens / 20)));
     }
     // The 32x32 kernel serves the two-heads layout; its V^T image keys are in
     // its own MFMA order.

@@ -413,3 +413,27 @@ def test_decode_single_layout(cuda, monkeypatch, pos):
         assert_attn_close(dev.out_f32(1)[0], want, f"decode step pos={pos}")
         dev.decode(1, pos)
         assert_attn_close(dev.out_f32(1)[0], want, f"decode pos={pos}")
+
+
+# The choices between the prefill kernels at their edges: 5 and 6 key chunks,
+# and 8 and 9 from an empty cache (16x16 / 32x32 kernel; a single tile: the split kernel), one tile per
+# workgroup with 1, 2, 4 and 8 key splits (49 chunks in 8 splits of 7: one
+# has none), as many tiles as CUs / KV heads (32) and one more (light
+# tiles beyond the first round, or pairs), 32 chunks per tile (the split kernel).
+@pytest.mark.parametrize("m,pos_base", [(129, 191), (129, 192), (512, 0), (513, 0), (32, 288), (32, 289), (31, 700), (33, 351), (64, 1000),
+                                        (64, 3072), (128, 3008), (65, 1300), (256, 1600), (255, 3000), (400, 2560), (512, 3300), (512, 100),
+                                        (1024, 33), (1025, 0), (1025, 64), (1056, 700), (64, 4032), (64, 4031)])
+def test_prefill_default_choices(cuda, m, pos_base):
+    _say(f"[prefill choices] m={m} pos_base={pos_base}")
+    cfg = layout.Config(n_layer=1)
+    sc = Scenario(cfg, max_seq=pos_base + m, m_tokens=m, seed=5 * m + pos_base)
+    _prefill_cache(sc, 0, pos_base, seed=178)
+    sc.oracle_q_norm_rope(pos_base)
+    sc.oracle_writeback(0, pos_base)
+    dev = DeviceScenario(sc, upload_kv=True)
+    dev.attention(0, pos_base, is_prefill=True)
+    rng = np.random.default_rng(3)
+    tokens = np.unique(np.concatenate([[0, 1, 31, 32, m - 1], np.arange(0, m, 64) + rng.integers(0, 64, (m + 63) // 64)]))
+    tokens = tokens[tokens < m]
+    want = sc.oracle_attention(0, pos_base, is_prefill=True, tokens=tokens)
+    assert_attn_close(dev.out_f32()[tokens], want, f"prefill m={m} pos_base={pos_base}")
