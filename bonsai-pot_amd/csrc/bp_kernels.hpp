@@ -162,7 +162,7 @@ struct MatvecArgs {
     uint32_t w_norm_off;
     float eps;
     uint32_t accumulate;      // plain / silu: y = f16(f32(y) + acc)
-    MatvecRange range[3];     // plain / silu: range[0] only; normed: multiples of 32 rows
+    MatvecRange range[3];     // plain / silu: range[0] only; normed: multiples of 16 rows
     uint32_t rows_per_wg;     // set by the launchers
     uint32_t stream_min_tiles;   // MFMA matvec: rows / 16 from which waves stream whole tiles
     uint32_t cu_count;

@@ -40,20 +40,29 @@ constexpr int kQ1Block = 128;
 constexpr int kHalfStride = 72;               // halves from one half-block to the next (64 + 8 pad)
 constexpr int kBlockHalves = 2 * kHalfStride; // one 128-element block in LDS
 
-// One lane's half of a (row, block): components 2h and 2h + 1, i.e. the
-// elements 4i + 2h and 4i + 2h + 1 for i = 0..31 in order, as one packed pair
-// of f16 accumulators. xh: the half-block of x.
-__device__ __forceinline__ h2v q1_half(const uint32_t q[4], const uint16_t* xh, uint32_t h) {
-    h2v c = {static_cast<_Float16>(0.0f), static_cast<_Float16>(0.0f)};
-    const uint32_t sh = 2 * h;
+// One lane's half of kRows (row, block)s of the same block: components 2h and
+// 2h + 1, i.e. the elements 4i + 2h and 4i + 2h + 1 for i = 0..31 in order, as
+// one packed pair of f16 accumulators per row. xh: the half-block of x, read
+// once for the rows.
+template <int kRows>
+__device__ __forceinline__ void q1_half(const uint4 (&q)[kRows], const uint16_t* xh, uint32_t h, h2v (&c)[kRows]) {
+    const uint32_t sh = 2 - 2 * h;
+#pragma unroll
+    for (int j = 0; j < kRows; j++) c[j] = h2v{static_cast<_Float16>(0.0f), static_cast<_Float16>(0.0f)};
 #pragma unroll
     for (int w = 0; w < 4; w++) {
-        const uint32_t nq = ~q[w];
-        // byte k of s[m] = 0x3C | (inverted bit 8k + p << 7), p = 2h + {0, 1, 4, 5}
-        const uint32_t s0 = __builtin_amdgcn_bitop3_b32(nq << (7 - sh), 0x80808080u, 0x3C3C3C3Cu, 0xEA);
-        const uint32_t s1 = __builtin_amdgcn_bitop3_b32(nq << (6 - sh), 0x80808080u, 0x3C3C3C3Cu, 0xEA);
-        const uint32_t s4 = __builtin_amdgcn_bitop3_b32(nq << (3 - sh), 0x80808080u, 0x3C3C3C3Cu, 0xEA);
-        const uint32_t s5 = __builtin_amdgcn_bitop3_b32(nq << (2 - sh), 0x80808080u, 0x3C3C3C3Cu, 0xEA);
+        uint32_t s[kRows][4];
+#pragma unroll
+        for (int j = 0; j < kRows; j++) {
+            // byte k of s[j][..] = 0x3C | (inverted bit 8k + p << 7), p = 2h + {0, 1, 4, 5};
+            // doublings by an add, which issues at twice the rate of a shift
+            const uint32_t b5 = (w == 0 ? q[j].x : w == 1 ? q[j].y : w == 2 ? q[j].z : q[j].w) << sh;
+            const uint32_t b4 = b5 + b5, b1 = b5 << 4, b0 = b1 + b1;
+            s[j][0] = __builtin_amdgcn_bitop3_b32(b0, 0x80808080u, 0x3C3C3C3Cu, 0xAE);   // (~a & b) | c
+            s[j][1] = __builtin_amdgcn_bitop3_b32(b1, 0x80808080u, 0x3C3C3C3Cu, 0xAE);
+            s[j][2] = __builtin_amdgcn_bitop3_b32(b4, 0x80808080u, 0x3C3C3C3Cu, 0xAE);
+            s[j][3] = __builtin_amdgcn_bitop3_b32(b5, 0x80808080u, 0x3C3C3C3Cu, 0xAE);
+        }
         const h8v xa = *reinterpret_cast<const h8v*>(xh + 16 * w);       // pairs i = 8w .. 8w + 3
         const h8v xb = *reinterpret_cast<const h8v*>(xh + 16 * w + 8);   // pairs i = 8w + 4 .. 8w + 7
 #pragma unroll
@@ -63,30 +72,35 @@ __device__ __forceinline__ h2v q1_half(const uint32_t q[4], const uint16_t* xh, 
 #pragma unroll
             for (int hh = 0; hh < 2; hh++) {   // pair m = 2k + hh of the word: bits 8k + 4hh + 2h + {0, 1}
                 const int m = 2 * k + hh;
-                const h2v sg = __builtin_bit_cast(h2v, hh == 0 ? __builtin_amdgcn_perm(s1, s0, sel)
-                                                                : __builtin_amdgcn_perm(s5, s4, sel));
                 const h2v xp = m < 4 ? h2v{xa[2 * m], xa[2 * m + 1]} : h2v{xb[2 * m - 8], xb[2 * m - 7]};
-                c = __builtin_elementwise_fma(sg, xp, c);
+#pragma unroll
+                for (int j = 0; j < kRows; j++) {
+                    const h2v sg = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(s[j][2 * hh + 1], s[j][2 * hh], sel));
+                    c[j] = __builtin_elementwise_fma(sg, xp, c[j]);
+                }
             }
         }
     }
-    return c;
 }
 
-// Weights of one lane's (row, block) in a tile: 16 qs bytes and the f16 scale.
+// Weights of one lane in a tile: 16 qs bytes and the f16 scale of kRows rows.
+template <int kRows>
 struct WTile {
-    uint4 q;
-    uint16_t d;
-    bool ok;
+    uint4 q[kRows];
+    uint16_t d[kRows];
 };
 
-// Tile t of a workgroup: rows 8 (t / tcols) .. + 7, blocks 4 (t % tcols) .. + 3;
-// lane = (row slot lane >> 3, block (lane >> 1) & 3, half lane & 1). A wave
-// walks tiles wave, wave + n_wave, ...; it keeps the tile's (row group, block
-// group) in scalar registers and steps them without a division.
+// Tile t of a workgroup: kTR rows (slots) by 32 / kTR blocks by 2 halves, rows
+// kTR kRows (t / tcols) .. + kTR kRows - 1, blocks from 32 / kTR (t % tcols) on; a
+// lane's kRows rows are kTR apart. A wave walks tiles wave, wave + n_wave, ...; it keeps the tile's
+// (row group, block group) in scalar registers and steps them without a division.
 struct TilePos {
     uint32_t tile, rq, col;   // wave-uniform
 };
+template <int kTR>
+__device__ __forceinline__ uint32_t tile_row(int lane) { return static_cast<uint32_t>(lane) / (64 / kTR); }
+template <int kTR>
+__device__ __forceinline__ uint32_t tile_block(int lane) { return (lane >> 1) & (32 / kTR - 1); }
 __device__ __forceinline__ void tile_step(TilePos& p, uint32_t n_wave, uint32_t tcols) {
     p.tile += n_wave;
     p.col += n_wave;
@@ -96,18 +110,20 @@ __device__ __forceinline__ void tile_step(TilePos& p, uint32_t n_wave, uint32_t 
     }
 }
 
-// Weights of one lane's (row, block) in a tile. Loads are unconditional (the
-// row and block clamped into range), so no lane branches around them; `ok`
-// says whether the lane's (row, block) exists.
-__device__ __forceinline__ WTile load_tile(const MatvecArgs& a, const TilePos& p, uint32_t n_tiles, uint32_t nb,
-                                           uint32_t n_here, uint32_t rbase, uint32_t d_off, uint32_t qs_off, int lane) {
-    WTile w;
-    const uint32_t r = p.rq * 8 + (lane >> 3), b = p.col * 4 + ((lane >> 1) & 3);
-    w.ok = p.tile < n_tiles && r < n_here && b < nb;
-    const uint32_t rc = min(r, n_here - 1), bc = min(b, nb - 1);
-    const uint32_t rb = (rbase + rc) * nb + bc;
-    w.q = *reinterpret_cast<const uint4*>(a.weights + qs_off + 16 * rb);
-    w.d = *reinterpret_cast<const uint16_t*>(a.weights + d_off + 2 * rb);
+// Weights of one lane in a tile. Loads are unconditional (rows and block
+// clamped into range), so no lane branches around them.
+template <int kTR, int kRows>
+__device__ __forceinline__ WTile<kRows> load_tile(const MatvecArgs& a, const TilePos& p, uint32_t nb, uint32_t n_here,
+                                                  uint32_t rbase, uint32_t d_off, uint32_t qs_off, int lane) {
+    WTile<kRows> w;
+    const uint32_t b = min(p.col * (32 / kTR) + tile_block<kTR>(lane), nb - 1);
+#pragma unroll
+    for (int j = 0; j < kRows; j++) {
+        const uint32_t r = min((p.rq * kRows + j) * kTR + tile_row<kTR>(lane), n_here - 1);
+        const uint32_t rb = (rbase + r) * nb + b;
+        w.q[j] = *reinterpret_cast<const uint4*>(a.weights + qs_off + 16 * rb);
+        w.d[j] = *reinterpret_cast<const uint16_t*>(a.weights + d_off + 2 * rb);
+    }
     return w;
 }
 
@@ -123,13 +139,13 @@ __device__ __forceinline__ void stage8(uint16_t* x_sh, uint32_t e, h8v r) {
 // kMode: 0 plain (x = act), 1 silu (x = f16(silu(gate)) * up), 2 normed
 // (x = act * w_norm, scale d * inv_rms, up to 3 row ranges).
 //
-// A workgroup owns rows_per_wg rows (its first weight loads are issued before
-// anything else). Pass 1 stages x. Pass 2: its waves share the tiles of those
-// rows (8 rows x 4 blocks x 2 halves each) and put each block's f32 term
+// A workgroup owns rows_per_wg rows, a multiple of kTR kRows (its first weight
+// loads are issued before anything else). Pass 1 stages x. Pass 2: its waves share
+// the tiles of those rows (kTR kRows rows x 32 / kTR blocks x 2 halves each) and put each block's f32 term
 // d * sum in LDS. Pass 3: thread (row, t) adds its terms t, t + 8, ... in order
 // and the 8 row lanes combine by the xor 1, 2, 4 butterfly.
-template <int kMode>
-__global__ __launch_bounds__(kMvMaxThreads) void matvec_q1_0_kernel(MatvecArgs a) {
+template <int kMode, int kTR, int kRows>
+__global__ __launch_bounds__(kRows == 1 ? kMvMaxThreads : 512) void matvec_q1_0_kernel(MatvecArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint16_t x_sh[];
     __shared__ float red_sh[4];
     const int t = threadIdx.x, n_thr = blockDim.x;
@@ -154,14 +170,14 @@ __global__ __launch_bounds__(kMvMaxThreads) void matvec_q1_0_kernel(MatvecArgs a
     }
     const uint32_t n_here = min(rows, a.n_total - row0);   // rows of this workgroup that exist
 
-    const uint32_t tcols = (nb + 3) / 4;
-    const uint32_t n_tiles = (rows / 8) * tcols;
+    const uint32_t tcols = (nb + 32 / kTR - 1) / (32 / kTR);
+    const uint32_t n_tiles = rows / (kTR * kRows) * tcols;
     TilePos pos = {static_cast<uint32_t>(wave), 0u, static_cast<uint32_t>(wave)};   // (rq, col) = divmod(wave, tcols)
     while (pos.col >= tcols) {   // no division: wave < 16, usually < tcols
         pos.col -= tcols;
         ++pos.rq;
     }
-    WTile cur = load_tile(a, pos, n_tiles, nb, n_here, rbase, d_off, qs_off, lane);   // in flight during pass 1
+    WTile<kRows> cur = load_tile<kTR, kRows>(a, pos, nb, n_here, rbase, d_off, qs_off, lane);   // in flight during pass 1
 
     // ---- pass 1: stage x (f16) into LDS, 8 elements at a time --------------------
     float ssq = 0.0f;
@@ -221,18 +237,28 @@ __global__ __launch_bounds__(kMvMaxThreads) void matvec_q1_0_kernel(MatvecArgs a
     while (pos.tile < n_tiles) {
         TilePos nxt_pos = pos;
         tile_step(nxt_pos, n_wave, tcols);
-        const WTile nxt = load_tile(a, nxt_pos, n_tiles, nb, n_here, rbase, d_off, qs_off, lane);
-        const uint32_t r = pos.rq * 8 + (lane >> 3), b = min(pos.col * 4 + ((lane >> 1) & 3), nb - 1);
-        const uint32_t q[4] = {cur.q.x, cur.q.y, cur.q.z, cur.q.w};
-        // both lanes of a pair are valid or invalid together; the lane exchange is
-        // executed by all lanes
-        const h2v c = q1_half(q, x_sh + b * kBlockHalves + h * kHalfStride, h);
-        const h2v c23 = __builtin_bit_cast(h2v, lane_xor<1>(__builtin_bit_cast(uint32_t, c)));
-        if (cur.ok && h == 0) {
-            const _Float16 sum = ((c.x + c.y) + c23.x) + c23.y;   // f16 adds, in this order
-            float d = static_cast<float>(__builtin_bit_cast(_Float16, cur.d));
+        const WTile<kRows> nxt = load_tile<kTR, kRows>(a, nxt_pos, nb, n_here, rbase, d_off, qs_off, lane);
+        const uint32_t b0 = pos.col * (32 / kTR) + tile_block<kTR>(lane), b = min(b0, nb - 1);
+        // the lane exchange is executed by all lanes
+        h2v c[kRows];
+        q1_half<kRows>(cur.q, x_sh + b * kBlockHalves + h * kHalfStride, h, c);
+        // The pair's lane h keeps row j = h of two rows (one row: lane 0 keeps it).
+        h2v c23[kRows];
+#pragma unroll
+        for (int j = 0; j < kRows; j++) c23[j] = __builtin_bit_cast(h2v, lane_xor<1>(__builtin_bit_cast(uint32_t, c[j])));
+        if (b0 < nb && (kRows == 2 || h == 0)) {
+            h2v lo = c[0], hi = c23[0];   // components 0, 1 and 2, 3
+            uint16_t dj = cur.d[0];
+            if (kRows == 2 && h == 1) {
+                lo = c23[kRows - 1];
+                hi = c[kRows - 1];
+                dj = cur.d[kRows - 1];
+            }
+            const uint32_t r = (pos.rq * kRows + (kRows == 2 ? h : 0u)) * kTR + tile_row<kTR>(lane);
+            const _Float16 sum = ((lo.x + lo.y) + hi.x) + hi.y;   // f16 adds, in this order
+            float d = static_cast<float>(__builtin_bit_cast(_Float16, dj));
             if constexpr (kMode == 2) d = d * inv_rms;
-            terms[r * nb + b] = d * static_cast<float>(sum);
+            if (r < n_here) terms[r * nb + b] = d * static_cast<float>(sum);
         }
         cur = nxt;
         pos = nxt_pos;
@@ -240,8 +266,8 @@ __global__ __launch_bounds__(kMvMaxThreads) void matvec_q1_0_kernel(MatvecArgs a
     __syncthreads();
 
     // ---- pass 3: the 8 ordered lane sums of each row, then the butterfly ----------
-    if (t < static_cast<int>(rows * 8)) {
-        const uint32_t r = t >> 3, bt = t & 7;
+    for (uint32_t i = t; i < rows * 8; i += n_thr) {   // (a row's 8 lanes stay together)
+        const uint32_t r = i >> 3, bt = i & 7;
         float acc = 0.0f;
         if (r < n_here)
             for (uint32_t b = bt; b < nb; b += 8) acc = acc + terms[r * nb + b];
@@ -260,47 +286,73 @@ __global__ __launch_bounds__(kMvMaxThreads) void matvec_q1_0_kernel(MatvecArgs a
 
 hipError_t launch_matvec_q1_0(const MatvecArgs& args, int mode, hipStream_t s) {
     MatvecArgs a = args;
-    const uint32_t nb = a.k / kQ1Block, tcols = (nb + 3) / 4;
-    // Rows per workgroup and waves: one tile per wave while the whole grid
-    // fits on the GPU at once (8192 waves). The silu matvec stages an expensive
-    // x, so it shares each staging among 16 rows. The normed sum of squares is
-    // defined over 256 threads (4 waves at least).
-    // Larger grids stage x once for 32 rows (64 from 2048 workgroups of those on)
-    // and use 8 waves, a multiple of the CU's 4 SIMDs: with one tile row's 5 waves
-    // (k = 2560) the first SIMD of a CU got two waves of every workgroup. us before
-    // (16 rows, two tiles per wave) and now: 19456 x 2560 7.2, 7.05; 24576 x 4096
-    // 11.0, 9.9; 32000 x 2048 8.0, 7.7; 151936 x 2560 37, 28.6 (32 rows: 29.2).
-    // Several ranges: rows have to divide them (16 always does); and x and the
-    // terms have to fit 64 KB of LDS.
-    auto plan = [&](uint32_t rows) {
-        a.rows_per_wg = rows;
-        const uint32_t w = std::min(rows / 8 * tcols, 16u);
-        return mode == 2 && w < 4 ? 4u : w;
-    };
+    const uint32_t nb = a.k / kQ1Block, cus = a.cu_count;
     auto lds_bytes = [&](uint32_t rows) { return static_cast<size_t>(nb) * kBlockHalves * 2 + static_cast<size_t>(rows) * nb * 4; };
-    uint32_t waves;
+    auto div_up = [](uint64_t x, uint64_t y) { return static_cast<uint32_t>((x + y - 1) / y); };
+    auto launch = [&](auto kernel, uint32_t rows, uint32_t waves) {
+        a.rows_per_wg = rows;
+        hipLaunchKernelGGL(kernel, dim3(div_up(a.n_total, rows)), dim3(64 * waves), lds_bytes(rows), s, a);
+        return hipGetLastError();
+    };
+
+    // Rows and waves per workgroup; us measured with all weights in turn.
     if (mode == 1) {
-        waves = plan(16);
-    } else {
-        waves = plan(8);
-        if (((a.n_total + 7) / 8) * waves > 8192) {
-            uint32_t rows = a.n_total >= 64 * 2048 ? 64 : 32;
-            const bool one_range = a.range[0].n == a.n_total;
-            while (rows > 16 && ((!one_range && (a.range[0].n % rows || a.range[1].n % rows)) || lds_bytes(rows) > 65536)) rows /= 2;
-            a.rows_per_wg = rows;
-            waves = rows == 16 ? 4 : 8;
+        // The silu matvec stages an expensive x: one workgroup per CU (or as few
+        // as keep it to 32 rows), so that no CU stages twice or idles, in tiles of
+        // 2 rows: 2560 x 9728 10 rows 6.52 (16 rows on 160 CUs 7.11, 8 rows 8.82),
+        // 2048 x 6144 5.26 -> 4.78, 1024 x 6144 5.07 -> 4.40; 4096 x 12288 (16 rows
+        // either way) 8.19 and 8.24. 16 waves where staging takes more than 12
+        // (2560 x 9728: 8 waves 6.79; 2048 x 6144: 16 waves 4.87).
+        // Below k = 3072 the staging is cheap and 16 blocks fill badly: 16 rows there
+        // (1024 x 2048 3.07, 4096 x 1024 2.87, tiles of 2 rows 3.20 and 3.18).
+        if (nb < 24) return launch(matvec_q1_0_kernel<1, 8, 1>, 16, std::min(2 * div_up(nb, 4), 16u));
+        const uint32_t rows = 2 * div_up(a.n_total, 2ull * cus * div_up(a.n_total, 32ull * cus));
+        return launch(matvec_q1_0_kernel<1, 2, 1>, rows, a.k > 6144 ? 16 : 8);
+    }
+    if (mode == 0 && nb >= 32 && nb % 8 == 0 && a.n_total <= 24 * cus) {
+        // Long rows, few of them: one workgroup per CU here too, tiles of 4 rows
+        // (2560 x 4096 4.23 -> 3.97, 4096 x 4096 4.40 -> 4.31, 1024 x 4096 3.24 ->
+        // 3.14; with k = 2048 the smaller workgroups below are as fast).
+        const uint32_t rows = 4 * div_up(a.n_total, 4 * cus), tiles = rows / 4 * (nb / 8);
+        return launch(matvec_q1_0_kernel<0, 4, 1>, rows, std::min(tiles, 16u));
+    }
+    // Up to 3 workgroups of 8 rows per CU: one tile per wave. Larger grids: each
+    // workgroup stages x again, about the work of 4 rows, and the busiest CU gets
+    // ceil(workgroups / CUs) of them, so the rows with the least of that times
+    // (rows + 4). Several ranges: rows have to divide them (16 always does), and x
+    // and the terms fit 64 KB of LDS. By 16 / 32 / 64 rows: 12288 x 2048 4.68 /
+    // 5.11 / 5.04 (8 rows 5.18), 19456 x 2560 6.9 / 6.9 / 7.2, 16384 x 2560 5.94 /
+    // 5.68 / 5.51, 24576 x 4096 9.95 / 9.31 / 10.3, 151936 x 2560 37 / 27.5 / 26.8.
+    // Waves are a multiple of the CU's 4 SIMDs (with one tile row's 5 at k = 2560
+    // the first SIMD gets two waves of every workgroup); the normed sum of squares
+    // is defined over 256 threads (4 waves at least).
+    const uint32_t tcols = (nb + 3) / 4;
+    uint32_t rows = 8;
+    if (a.n_total > 24 * cus) {
+        const bool one_range = a.range[0].n == a.n_total;
+        uint64_t best = ~0ull;
+        for (uint32_t r : {16u, 32u, 64u}) {
+            if (r > 16 && ((!one_range && (a.range[0].n % r || a.range[1].n % r)) || lds_bytes(r) > 65536)) continue;
+            const uint64_t cost = static_cast<uint64_t>(div_up(a.n_total, static_cast<uint64_t>(r) * cus)) * (r + 4);
+            if (cost <= best) best = cost, rows = r;
         }
     }
-    const uint32_t n_wg = (a.n_total + a.rows_per_wg - 1) / a.rows_per_wg;
-    const size_t lds = lds_bytes(a.rows_per_wg);
-    const dim3 block(64 * waves);
-    if (mode == 0)
-        hipLaunchKernelGGL(matvec_q1_0_kernel<0>, dim3(n_wg), block, lds, s, a);
-    else if (mode == 1)
-        hipLaunchKernelGGL(matvec_q1_0_kernel<1>, dim3(n_wg), block, lds, s, a);
-    else
-        hipLaunchKernelGGL(matvec_q1_0_kernel<2>, dim3(n_wg), block, lds, s, a);
-    return hipGetLastError();
+    if (rows <= 16) {
+        const uint32_t waves = rows == 16 ? 4u : std::max(std::min(tcols, 16u), mode == 2 ? 4u : 1u);
+        return mode == 0 ? launch(matvec_q1_0_kernel<0, 8, 1>, rows, waves) : launch(matvec_q1_0_kernel<2, 8, 1>, rows, waves);
+    }
+    // Two rows per lane (x read from LDS once for both, two independent chains:
+    // 151936 x 2560 28.6 -> 26.8, 24576 x 4096 9.65 -> 9.31) unless 32 rows then
+    // keep the waves busy for longer (k = 2560: 20 tiles on 8 waves 5.68, 10 double
+    // ones 5.98). 4 waves for grids of many workgroups, 8 otherwise (151936 x 2560
+    // 26.8 and 27.4; 32000 x 2048 7.50 and 7.21); the normed staging is done by 4
+    // waves, so there from 2 workgroups per CU (24576 x 4096 9.31 and 9.64).
+    const uint32_t doubles = rows / 16 * tcols, n_wg = div_up(a.n_total, rows);
+    if (rows == 64 || 2 * ((doubles + 7) / 8) <= (2 * doubles + 7) / 8) {
+        const uint32_t waves = n_wg >= 4 * cus || (mode == 2 && rows == 32 && n_wg >= 2 * cus) ? 4 : 8;
+        return mode == 0 ? launch(matvec_q1_0_kernel<0, 8, 2>, rows, waves) : launch(matvec_q1_0_kernel<2, 8, 2>, rows, waves);
+    }
+    return mode == 0 ? launch(matvec_q1_0_kernel<0, 8, 1>, rows, 8) : launch(matvec_q1_0_kernel<2, 8, 1>, rows, 8);
 }
 
 uint32_t matvec_max_k() { return 16384; }

@@ -489,3 +489,47 @@ def test_matvec_fused_normed_large_grids(cuda, monkeypatch, sizes):
                                                 [(d + 2 * lo * (k // 128), q + 16 * lo * (k // 128), c, o + lo)])
     torch.cuda.synchronize()
     assert torch.equal(got_d, want_d)
+
+
+# The f16-order kernel's plan at its edges: 16 rows (from 24 rows per CU on), 32
+# with one and two rows per lane, 64; long rows in tiles of 4 rows; rows past the
+# last whole workgroup, blocks past the last whole tile.
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k,acc", [(6144, 1152, 0), (6145, 1152, 1), (8192 - 3, 2048, 0), (8192, 2560, 1), (11000, 640, 0),
+                                     (16384, 1024, 0), (16389, 2048, 1), (1, 4096, 0), (1027, 4096, 1), (2560, 4096, 1),
+                                     (3000, 5120, 0), (2050, 4224, 0), (514, 16384, 0)])
+def test_matvec_plan_choices(cuda, monkeypatch, n, k, acc):
+    test_matvec_large_grids(cuda, monkeypatch, n, k, acc)
+
+
+# The silu matvec in tiles of 2 rows x 16 blocks: from 2 rows per workgroup to 32
+# and a second round of workgroups, odd rows, 8 and 16 waves.
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k,acc", [(1, 3072, 0), (513, 3072, 1), (1024, 3072, 0), (1025, 3200, 1), (2560, 2944, 0),
+                                     (300, 6144, 0), (301, 6272, 1), (100, 16384, 0), (8192, 3072, 0), (8193, 3072, 1)])
+def test_matvec_silu_plan_choices(cuda, monkeypatch, n, k, acc):
+    test_matvec_silu(cuda, monkeypatch, "f16", n, k, acc)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes,k", [((8192, 16384), 2048), ((8192 + 16, 16384), 2048), ((4096, 2048, 64), 1024), ((9728, 9728), 640),
+                                     ((16384,), 1152)])
+def test_matvec_fused_normed_plan_choices(cuda, monkeypatch, sizes, k):
+    """Each range must be the product that 1024 of its rows alone give (small grids, bit-exact above)."""
+    _say(f"[matvec normed plan] sizes={sizes} k={k}")
+    rng = np.random.default_rng(sum(sizes))
+    buf, offs = _weights(rng, [(n, k) for n in sizes])
+    total = sum(sizes)
+    act = _f16(rng.standard_normal(k + total + 64))
+    norms = _f16(1 + 0.1 * rng.standard_normal(k))
+    m = _model(monkeypatch, "f16")
+    w_d, n_d = _dev(buf), _dev(norms)
+    at = np.concatenate([[0], np.cumsum(sizes)[:-1]]) + k + 8
+    got_d, want_d = _dev(act), _dev(act)
+    m.dispatch_matvec_q1_0_fused_normed(w_d.data_ptr(), got_d.data_ptr(), n_d.data_ptr(), k, 0, 0,
+                                        [(d, q, n, int(o)) for (d, q), n, o in zip(offs, sizes, at)])
+    for (d, q), n, o in zip(offs, sizes, at):
+        for r in range(0, n, 1024):   # 1024 rows at a time: 8 rows a workgroup, one tile a wave
+            m.dispatch_matvec_q1_0_fused_normed(w_d.data_ptr(), want_d.data_ptr(), n_d.data_ptr(), k, 0, 0,
+                                                [(d + 2 * r * (k // 128), q + 16 * r * (k // 128), min(1024, n - r), int(o) + r)])
+    assert np.array_equal(_host(got_d), _host(want_d))
