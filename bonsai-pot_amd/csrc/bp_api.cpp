@@ -48,7 +48,7 @@ struct bp_model {
     uint32_t decode_wide_min_rows;
     uint32_t prefill_hpw;   // 0 = by grid size; 2 = prefill32_kernel, 1 = the one-head 16x16 kernels
     uint32_t prefill_waves; // 0 = by grid size, else 4 or 8 waves per workgroup at 1 head per wave
-    uint32_t prefill_ksplit;   // 0 = by grid size, else the key split count of the 4-wave layout
+    uint32_t prefill_ksplit;   // 0 = by grid size, else prefill_split_kernel's split count
     int matvec_arith;        // Q1_0 matvecs: 0 auto, 1 (default) f16 sums in the reference's order, 2 i8 MFMA
     uint32_t matvec_stream_min_tiles;
     bool lost;

@@ -210,17 +210,18 @@ void decode_plan(uint32_t n_rows, uint32_t n_kv_head, int cu_count, uint32_t min
                  uint32_t wide_min_rows, uint32_t* split_len, uint32_t* n_splits, uint32_t* heads_per_wg);
 uint32_t decode_max_splits();
 uint32_t decode_partial_stride();   // floats per (head, split) partial
-// Plain decode (q already normalized, cache row already written): one launch
-// when n_splits == 1, else split pass + merge pass.
+// Plain decode (q already normalized, cache row already written): one launch in
+// the single layout or when n_splits == 1, else split pass + merge pass.
 hipError_t launch_decode(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s);
-// Fused decode step: split pass (with q norm + row writeback) + merge pass.
+// Fused decode step: split pass (with q norm + row writeback) + merge pass, or
+// the single layout's one launch.
 hipError_t launch_decode_step(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s);
 hipError_t launch_prefill(const PrefillArgs& a, uint32_t n_kv_head, hipStream_t s);
 // Whether the launches of launch_prefill (step = false) or launch_prefill_step
 // (step = true) for these arguments fit HIP's grid limits (y, z <= 65535).
 bool prefill_grid_fits(const PrefillArgs& a, bool step);
 // The fused prefill step: preparation pass (in place of the dequantization
-// pass) and attention, 2 launches; with prep_only the first launch alone.
+// pass) and attention, 2 launches (3 with a key split); with prep_only the first launch alone.
 hipError_t launch_prefill_step(const PrefillArgs& a, const PrefillStepArgs& w, uint32_t n_kv_head, hipStream_t s,
                                bool prep_only);
 

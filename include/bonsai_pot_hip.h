@@ -10,9 +10,9 @@
  *   bp_dispatch_kv_writeback_fused   <- dispatch_kv_writeback_fused  src/forward.rs:359-388
  *   bp_dispatch_attention_decode     <- split+merge block in layer_post_kv_in_pass
  *                                       src/forward.rs:820-857
- *   bp_dispatch_attention_decode_step <- the three above for one token (fused, 2 launches)
+ *   bp_dispatch_attention_decode_step <- the three above for one token (fused, 1 or 2 launches)
  *   bp_dispatch_attention            <- dispatch_attention           src/forward.rs:501-532
- *   bp_dispatch_attention_prefill_step <- q_norm_rope + kv_writeback + attention for m tokens (fused, 2 launches)
+ *   bp_dispatch_attention_prefill_step <- q_norm_rope + kv_writeback + attention for m tokens (fused, 2 or 3 launches)
  *   bp_dispatch_matvec_q1_0          <- dispatch_matvec_q1_0         src/forward.rs:212-241
  *   bp_dispatch_matvec_q1_0_silu     <- dispatch_matvec_q1_0_silu    src/forward.rs:243-282
  *   bp_dispatch_matvec_q1_0_fused_normed <- dispatch_matvec_q1_0_fused_normed
@@ -128,7 +128,7 @@ bp_status bp_dispatch_attention_decode(bp_model* model, void* act, uint32_t q_of
                                        uint32_t out_off, uint32_t layer_il, uint32_t pos);
 
 /* One whole attention decode step for one layer at step position `pos`, in
- * two launches instead of the reference's four dispatches: the same results as
+ * at most two launches instead of the reference's four dispatches: the same results as
  *   bp_dispatch_q_norm_rope_fused(act, w_norms, q_off, w_q_norm_off, pos, 1)
  *   bp_dispatch_kv_writeback_fused(act, w_norms, k_cur_off, v_cur_off, w_k_norm_off, layer_il, pos, 1)
  *   bp_dispatch_attention_decode(act, q_off, out_off, layer_il, pos)
@@ -154,7 +154,7 @@ bp_status bp_dispatch_attention(bp_model* model, void* act, uint32_t q_off, uint
                                 uint32_t is_prefill);
 
 /* One whole causal prefill-attention step for one layer: m_tokens tokens at
- * cache rows [pos, pos+m_tokens), in two launches instead of four, with the
+ * cache rows [pos, pos+m_tokens), in two or three launches instead of four, with the
  * same results as
  *   bp_dispatch_q_norm_rope_fused(act, w_norms, q_off, w_q_norm_off, pos, m_tokens)
  *   bp_dispatch_kv_writeback_fused(act, w_norms, k_cur_off, v_cur_off, w_k_norm_off, layer_il, pos, m_tokens)
