@@ -628,7 +628,8 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(
 }  // namespace
 
 void decode_plan(uint32_t n_rows, uint32_t n_kv_head, int cu_count, uint32_t min_split_rows,
-                 uint32_t wide_min_rows, uint32_t* split_len, uint32_t* n_splits, uint32_t* heads_per_wg) {
+                 uint32_t wide_min_rows, bool may_single, uint32_t* split_len, uint32_t* n_splits,
+                 uint32_t* heads_per_wg, uint32_t* single) {
     // Layout: 4 KV heads per workgroup from wide_min_rows rows on (long
     // contexts: rows are read whole), else 1 (short contexts: 4 waves per head
     // keep each wave's chain short). Then enough workgroups to fill every CU
@@ -649,7 +650,10 @@ void decode_plan(uint32_t n_rows, uint32_t n_kv_head, int cu_count, uint32_t min
     // 8.9, as split + merge 8.0 / 7.7 / 7.9 / 7.9 (calls in a row; graph replays
     // at 300 and 500 6.6 and 9.0 against 6.7 and 7.1). A batch costs a wave about
     // 1 us: two waves a SIMD issue an instruction every three cycles each.
-    if (h == 1 && n_rows <= 3 * min_split_rows) {
+    // Not where a workgroup's output could land in what another still reads
+    // (may_single): the split layout stores it in the second launch.
+    *single = may_single && h == 1 && n_rows <= 3 * min_split_rows ? 1u : 0u;
+    if (*single) {
         *split_len = (n_rows + 15) / 16 * 16;
         *n_splits = 1;
         *heads_per_wg = 1;
@@ -666,13 +670,10 @@ void decode_plan(uint32_t n_rows, uint32_t n_kv_head, int cu_count, uint32_t min
 uint32_t decode_max_splits() { return kMaxSplits; }
 uint32_t decode_partial_stride() { return kPartStride; }
 
-// One split of one KV head per workgroup: the single layout, no merge pass.
-static bool decode_single(const DecodeArgs& a) { return a.n_splits == 1 && a.heads_per_wg == 1; }
-
 template <bool kFused>
 static void launch_split(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s) {
     const uint32_t z = (a.n_splits + 7) / 8;
-    if (decode_single(a))
+    if (a.single)
         hipLaunchKernelGGL((decode_split_kernel<kFused, 1, true>), dim3(1, n_kv_head, 1),
                            dim3(SplitShape<1, true>::kThreads), 0, s, a);
     else if (a.heads_per_wg == 4)
@@ -705,14 +706,14 @@ static void launch_merge(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s)
 
 hipError_t launch_decode(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s) {
     launch_split<false>(a, n_kv_head, s);
-    if (!decode_single(a))
+    if (!a.single)
         launch_merge<false>(a, n_kv_head, s);
     return hipGetLastError();
 }
 
 hipError_t launch_decode_step(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s) {
     launch_split<true>(a, n_kv_head, s);
-    if (!decode_single(a))
+    if (!a.single)
         launch_merge<true>(a, n_kv_head, s);
     return hipGetLastError();
 }

@@ -153,8 +153,21 @@ bp::KvView kv_view(const bp_model* m, const uint8_t* buf, uint32_t il) {
 
 constexpr uint32_t kMaxGridY = 65535;
 
+// Whether na f16 elements at a and nb at b share memory.
+bool overlap(const uint16_t* a, uint64_t na, const uint16_t* b, uint64_t nb) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + 2 * nb && y < x + 2 * na;
+}
+
+// The single decode layout reads and writes act in one launch, a workgroup per KV
+// head: out may be q itself (each workgroup reads its own heads before it stores
+// them), but not lie across other heads' q.
+bool decode_may_single(const uint16_t* q, const uint16_t* out, uint32_t q_dim) {
+    return q == out || !overlap(q, q_dim, out, q_dim);
+}
+
 bp::DecodeArgs decode_args(const bp_model* m, void* act, uint32_t q_off, uint32_t out_off, uint32_t il,
-                           uint32_t n_rows) {
+                           uint32_t n_rows, bool may_single) {
     bp::DecodeArgs a{};
     a.q = static_cast<const uint16_t*>(act) + q_off;
     a.out = static_cast<uint16_t*>(act) + out_off;
@@ -163,8 +176,9 @@ bp::DecodeArgs decode_args(const bp_model* m, void* act, uint32_t q_off, uint32_
     a.partials = m->partials;
     a.kv_dim = m->kv_dim;
     a.n_rows = n_rows;
-    bp::decode_plan(n_rows, m->cfg.n_kv_head, m->cu_count, m->decode_min_split_rows,
-                    m->decode_wide_min_rows, &a.split_len, &a.n_splits, &a.heads_per_wg);
+    bp::decode_plan(n_rows, m->cfg.n_kv_head, m->cu_count, m->decode_min_split_rows, m->decode_wide_min_rows,
+                    may_single && decode_may_single(a.q, a.out, m->q_dim), &a.split_len, &a.n_splits,
+                    &a.heads_per_wg, &a.single);
     a.scale = 1.0f / std::sqrt(static_cast<float>(m->cfg.head_dim));   // src/forward.rs:838
     return a;
 }
@@ -463,7 +477,7 @@ bp_status bp_dispatch_attention_decode(bp_model* m, void* act, uint32_t q_off, u
                     m->max_seq);
     if ((q_off & 7u) || (out_off & 3u))
         return fail(BP_ERR_INVALID_ARG, "q_off must be a multiple of 8 and out_off of 4 (aligned f16 rows)");
-    bp::DecodeArgs a = decode_args(m, act, q_off, out_off, layer_il, pos + 1);   // src/forward.rs:822
+    bp::DecodeArgs a = decode_args(m, act, q_off, out_off, layer_il, pos + 1, true);   // src/forward.rs:822
     if (static_cast<uint64_t>(a.n_splits) * m->cfg.n_head * bp::decode_partial_stride() > m->partials_floats)
         return fail(BP_ERR_CONFIG, "internal: partials scratch too small for %u splits", a.n_splits);
     return hip_check(m, bp::launch_decode(a, m->cfg.n_kv_head, m->stream), "attention_decode launch");
@@ -484,12 +498,21 @@ bp_status bp_dispatch_attention_decode_step(bp_model* m, void* act, const void* 
     if ((out_off & 3u))
         return fail(BP_ERR_INVALID_ARG, "out_off must be a multiple of 4 (8-byte aligned f16 rows)");
     // The split pass streams rows [0, pos); row `pos` is written and added in-kernel.
-    bp::DecodeArgs a = decode_args(m, act, q_off, out_off, layer_il, pos);
-    a.q_act = static_cast<uint16_t*>(act) + q_off;
+    // out may take the place of k_cur / v_cur, which are dead once the row is written:
+    // then every workgroup has to read before one stores out (or the normalized q).
+    uint16_t* const x = static_cast<uint16_t*>(act);
+    const uint16_t* const w = static_cast<const uint16_t*>(w_norms);
+    const struct { const uint16_t* at; uint32_t n; } reads[] = {{x + k_cur_off, m->kv_dim}, {x + v_cur_off, m->kv_dim},
+        {w + w_q_norm_off, m->cfg.head_dim}, {w + w_k_norm_off, m->cfg.head_dim}};
+    bool may_single = true;
+    for (const auto& r : reads)
+        may_single = may_single && !overlap(x + out_off, m->q_dim, r.at, r.n) && !overlap(x + q_off, m->q_dim, r.at, r.n);
+    bp::DecodeArgs a = decode_args(m, act, q_off, out_off, layer_il, pos, may_single);
+    a.q_act = x + q_off;
     a.q_norm = m->q_norm;
-    a.k_cur = static_cast<const uint16_t*>(act) + k_cur_off;
-    a.v_cur = static_cast<const uint16_t*>(act) + v_cur_off;
-    a.w_norms = static_cast<const uint16_t*>(w_norms);
+    a.k_cur = x + k_cur_off;
+    a.v_cur = x + v_cur_off;
+    a.w_norms = w;
     a.rope_cs = m->rope_cs;
     a.w_q_off = w_q_norm_off;
     a.w_k_off = w_k_norm_off;
@@ -970,7 +993,8 @@ bp_status bp_attention_decode_noalloc(const bp_config* cfg, void* kv_k, void* kv
     a.kv_dim = kv_dim;
     a.n_rows = pos + 1;   // src/forward.rs:822
     bp::decode_plan(a.n_rows, cfg->n_kv_head, d->cu_count, bp::kDecodeMinSplitRows, bp::kDecodeWideMinRows,
-                    &a.split_len, &a.n_splits, &a.heads_per_wg);
+                    decode_may_single(a.q, a.out, cfg->n_head * cfg->head_dim), &a.split_len, &a.n_splits,
+                    &a.heads_per_wg, &a.single);
     a.scale = 1.0f / std::sqrt(static_cast<float>(cfg->head_dim));   // src/forward.rs:838
     if (static_cast<uint64_t>(a.n_splits) * cfg->n_head * bp::decode_partial_stride() > kNoAllocScratchFloats)
         return fail(BP_ERR_CONFIG, "noalloc decode: %u query heads x %u splits exceed the %llu-float scratch",

@@ -61,13 +61,14 @@ struct DecodeArgs {
     float* partials;          // n_head * n_splits * decode_partial_stride() floats: o rows, then (m, l)
     uint32_t kv_dim;
     uint32_t n_rows;          // rows streamed by the split pass: [0, n_rows)
-    uint32_t split_len;       // rows per workgroup, multiple of 32
+    uint32_t split_len;       // rows per workgroup, multiple of 32 (single layout: 16)
     uint32_t n_splits;        // >= 1
     uint32_t heads_per_wg;    // split-pass layout: 1 or 4 KV heads per workgroup
     float scale;
     // Fused decode step only (q_norm_rope + kv_writeback of row `pos` + attention
     // over rows [0, pos]): the split pass normalizes q itself and writes cache row
-    // `pos`; the merge pass adds that row and stores the normalized q into act.
+    // `pos`; the merge pass (the one launch of the single layout) adds that row and
+    // stores the normalized q into act.
     uint16_t* q_act;          // act + q_off (receives the normalized q)
     uint16_t* q_norm;         // scratch [n_head][128] f16
     const uint16_t* k_cur;    // act + k_cur_off: [n_kv_head][128]
@@ -77,6 +78,7 @@ struct DecodeArgs {
     uint64_t w_q_off, w_k_off;
     uint32_t pos;
     float eps;
+    uint32_t single;          // 1: the single layout, one launch (n_splits = heads_per_wg = 1)
 };
 
 struct PrefillArgs {
@@ -205,13 +207,15 @@ hipError_t launch_q_norm_rope(const QNormRopeArgs& a, uint32_t n_head, uint32_t 
 hipError_t launch_kv_writeback(const KvWritebackArgs& a, uint32_t n_kv_head, uint32_t m_tokens,
                                hipStream_t s);
 // Split-K plan of a decode over n_rows rows (1 <= n_splits <= decode_max_splits())
-// and the split pass's layout (heads_per_wg = 4 from wide_min_rows rows on).
+// and the split pass's layout (heads_per_wg = 4 from wide_min_rows rows on), or
+// where may_single the single layout at the shortest contexts.
 void decode_plan(uint32_t n_rows, uint32_t n_kv_head, int cu_count, uint32_t min_split_rows,
-                 uint32_t wide_min_rows, uint32_t* split_len, uint32_t* n_splits, uint32_t* heads_per_wg);
+                 uint32_t wide_min_rows, bool may_single, uint32_t* split_len, uint32_t* n_splits,
+                 uint32_t* heads_per_wg, uint32_t* single);
 uint32_t decode_max_splits();
 uint32_t decode_partial_stride();   // floats per (head, split) partial
 // Plain decode (q already normalized, cache row already written): one launch in
-// the single layout or when n_splits == 1, else split pass + merge pass.
+// the single layout, else split pass + merge pass.
 hipError_t launch_decode(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s);
 // Fused decode step: split pass (with q norm + row writeback) + merge pass, or
 // the single layout's one launch.

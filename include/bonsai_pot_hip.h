@@ -134,7 +134,9 @@ bp_status bp_dispatch_attention_decode(bp_model* model, void* act, uint32_t q_of
  *   bp_dispatch_attention_decode(act, q_off, out_off, layer_il, pos)
  * i.e. src/forward.rs:796-804 + :618-628 + :820-857 for one token. act[q_off]
  * holds the raw (pre-norm) query and receives the normalized one; cache row
- * `pos` receives the new K/V; act[out_off] receives the attention output. */
+ * `pos` receives the new K/V; act[out_off] receives the attention output, which
+ * may lie over k_cur / v_cur or be q's own region (out_off == q_off): the launches
+ * are then as many as that order needs. */
 bp_status bp_dispatch_attention_decode_step(bp_model* model, void* act, const void* w_norms,
                                             uint32_t q_off, uint32_t k_cur_off, uint32_t v_cur_off,
                                             uint32_t out_off, uint32_t w_q_norm_off,
