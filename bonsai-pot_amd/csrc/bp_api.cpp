@@ -581,9 +581,15 @@ static bp_status prefill_args(bp_model* m, void* act, uint32_t q_off, uint32_t o
         //    rows 54, prefill32_kernel 69; 128 on 8192 52 and 51), and for a single
         //    tile (16 on 500 / 1000 rows 16.0 / 16.0, prefill32_kernel 20.1 / 20.9);
         //  * else prefill32_kernel.
+        // With out across q (neither apart nor q itself) the other two would store into
+        // what another workgroup still reads; the split kernel stores in its merge, so
+        // it takes those calls from 4 chunks per tile on.
         a.heads_per_wave = m->prefill_hpw != 0 ? m->prefill_hpw : 2u;
+        const uint64_t elems = static_cast<uint64_t>(m_tokens) * m->q_dim;
+        const bool across = a.q != a.out && overlap(a.q, elems, a.out, elems);
+        const uint64_t from = across ? 4ull * a.n_tiles : a.n_tiles == 1 ? 6 : 32ull * a.n_tiles;
         if (m->prefill_hpw != 2 && is_prefill && small && m->prefill_waves != 8 &&
-            (m->prefill_ksplit != 0 || chunks >= (a.n_tiles == 1 ? 6 : 32 * a.n_tiles))) {
+            (m->prefill_ksplit != 0 || chunks >= from)) {
             // one 8-wave workgroup per (KV head, key split, tile pair): enough splits
             // to give every CU a workgroup, at least 2 chunks each (a single tile: 1,
             // up to 16 splits; 16 tokens on 1000 rows: 8 splits 16.9, 16 16.0)

@@ -149,6 +149,7 @@ bp_status bp_dispatch_attention_decode_step(bp_model* model, void* act, const vo
  * is_prefill != 0 this is the reference's causal prefill from an empty cache;
  * pos > 0 is causal chunked prefill over an existing cache (the reference
  * reaches that result only one token at a time, src/forward.rs:914-967).
+ * The out region is q's own (out_off == q_off) or apart from it.
  * BP_ERR_CONFIG when the cache rows or tokens exceed the kernels' grid limits
  * (more than 65535 64-row chunks, or 65535 pairs of 32-token tiles). */
 bp_status bp_dispatch_attention(bp_model* model, void* act, uint32_t q_off, uint32_t out_off,

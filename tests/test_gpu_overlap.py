@@ -89,3 +89,31 @@ def test_decode_out_over_q(cuda, shift, launches, pos):
     dev.decode(1, pos)
     _, want = sc.oracle_decode(1, pos)
     assert_attn_close(dev.out_f32(1)[0], want, f"decode, out over q + {shift}, pos={pos}")
+
+
+@pytest.mark.parametrize("shift,launches", [(0, 2), (512, 3), (8, 3)])
+@pytest.mark.parametrize("m,pos", [(64, 448), (64, 576), (40, 500), (32, 288)])
+def test_prefill_step_out_over_q(cuda, m, pos, shift, launches):
+    """A short chunk over 4 to 11 key chunks per tile: out on q itself, and across
+    other heads' q, where the merge pass has to store it."""
+    _say(f"[overlap] prefill step out over q + {shift} m={m} pos={pos}")
+    cfg = layout.Config(n_layer=2)
+    sc = Scenario(cfg, max_seq=pos + m, m_tokens=m, seed=1700 + m + pos, w_std=0.1)
+    pre = Scenario(cfg, sc.max_seq, pos, seed=1701, with_q=False)
+    pre.oracle_writeback(1, 0)
+    sc.kv_k[:], sc.kv_v[:] = pre.kv_k, pre.kv_v
+    sc.out_off = sc.q_off + shift
+    if shift:   # out of the last token reaches into k, which the preparation pass has read by then
+        assert sc.out_off + m * cfg.q_dim <= sc.v_off
+    dev = DeviceScenario(sc, upload_kv=True)
+
+    def step():
+        dev.model.dispatch_attention_prefill_step(dev.act.data_ptr(), dev.w.data_ptr(), sc.q_off, sc.k_off, sc.v_off,
+                                                  sc.out_off, sc.w_q_off, sc.w_k_off, 1, pos, m)
+    assert _nodes(dev.model, step) == launches
+    step()
+    sc.oracle_q_norm_rope(pos)
+    sc.oracle_writeback(1, pos)
+    k, v = dev.kv_host()
+    assert np.array_equal(k, sc.kv_k) and np.array_equal(v, sc.kv_v), "cache bytes differ"
+    assert_attn_close(dev.out_f32(), sc.oracle_attention(1, pos), f"prefill step, out over q + {shift}, m={m} pos={pos}")
