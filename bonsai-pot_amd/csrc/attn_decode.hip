@@ -28,8 +28,8 @@
 //    into the B layout with v_perm_b32.
 //  * The row sets of a KV head are merged through LDS (log-sum-exp) into one
 //    partial (o[128], m, l) per query head. At the shortest contexts one
-//    workgroup of 8 waves takes a KV head's whole context (the single layout),
-//    adds row `pos` itself in the fused step and stores the output: no merge pass.
+//    workgroup takes a KV head's whole context (in the single layout of 8 waves it
+//    also adds row `pos` of the fused step) and stores the output: no merge pass.
 //
 // Merge pass (decode_merge_kernel) — one 64-lane workgroup per (query head,
 // 32-dim chunk): log-sum-exp over the splits (attention_merge.wgsl:85-129),
@@ -155,6 +155,8 @@ __global__ __launch_bounds__(Shape::kThreads, Shape::kWgPerCu) void decode_split
     if constexpr (kFused)
         asm volatile("" ::"s"(a.w_norms), "s"(a.rope_cs), "s"(a.pos), "s"(a.w_q_off), "s"(a.w_k_off),
                      "s"(a.k_cur), "s"(a.v_cur));
+    else
+        asm volatile("" ::"s"(a.no_merge));
     if (split >= a.n_splits) return;
     const uint32_t row0 = min(split * a.split_len, a.n_rows);
     const uint32_t row_end = min(row0 + a.split_len, a.n_rows);
@@ -492,6 +494,14 @@ __global__ __launch_bounds__(Shape::kThreads, Shape::kWgPerCu) void decode_split
         a.out[static_cast<uint64_t>(qhd) * kHeadDim + fd] = f2h(o[0] * (1.0f / L));
         return;
     } else {
+        if (!kFused && a.no_merge) {
+            const float inv_l = 1.0f / L;
+#pragma unroll
+            for (int k = 0; k < kE; k += 2)
+                *reinterpret_cast<uint32_t*>(a.out + static_cast<uint64_t>(qhd) * kHeadDim + fd + k) =
+                    static_cast<uint32_t>(f2h(o[k] * inv_l)) | (static_cast<uint32_t>(f2h(o[k + 1] * inv_l)) << 16);
+            return;
+        }
         float* part = part_o(a.partials, qhd, a.n_splits, split);
 #pragma unroll
         for (int k = 0; k + 1 < kE; k += 2) *reinterpret_cast<float2*>(part + fd + k) = make_float2(o[k], o[k + 1]);
@@ -627,15 +637,15 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(
 
 }  // namespace
 
-void decode_plan(uint32_t n_rows, uint32_t n_kv_head, int cu_count, uint32_t min_split_rows,
-                 uint32_t wide_min_rows, bool may_single, uint32_t* split_len, uint32_t* n_splits,
-                 uint32_t* heads_per_wg, uint32_t* single) {
+void decode_plan(DecodeArgs& a, uint32_t n_kv_head, int cu_count, uint32_t min_split_rows, uint32_t wide_min_rows,
+                 bool fused, bool may_one_launch) {
     // Layout: 4 KV heads per workgroup from wide_min_rows rows on (long
     // contexts: rows are read whole), else 1 (short contexts: 4 waves per head
     // keep each wave's chain short). Then enough workgroups to fill every CU
     // at 2 waves per SIMD, but at least min_split_rows rows each (fewer
     // partials at short context) and at most kMaxSplits splits; rows per split
     // are a multiple of one batch of all row sets.
+    const uint32_t n_rows = a.n_rows;
     const uint32_t h = n_rows >= wide_min_rows && n_kv_head % 4 == 0 ? 4 : 1;
     const uint32_t wg_per_cu = h == 1 ? SplitShape<1>::kWgPerCu : SplitShape<4>::kWgPerCu;
     const uint32_t batch_rows = 16u * (h == 1 ? SplitShape<1>::kRowSets : SplitShape<4>::kRowSets);
@@ -644,27 +654,28 @@ void decode_plan(uint32_t n_rows, uint32_t n_kv_head, int cu_count, uint32_t min
     uint32_t want = (target + groups - 1) / groups;
     if (want < 1) want = 1;
     if (want > kMaxSplits) want = kMaxSplits;
-    // Up to three batches per wave the whole context of a KV head goes to one
-    // workgroup (n_splits = 1: the single layout), because the merge pass costs a
-    // launch: us per fused step at 100 / 200 / 300 / 500 rows 5.3 / 5.8 / 6.5 /
-    // 8.9, as split + merge 8.0 / 7.7 / 7.9 / 7.9 (calls in a row; graph replays
-    // at 300 and 500 6.6 and 9.0 against 6.7 and 7.1). A batch costs a wave about
-    // 1 us: two waves a SIMD issue an instruction every three cycles each.
-    // Not where a workgroup's output could land in what another still reads
-    // (may_single): the split layout stores it in the second launch.
-    *single = may_single && h == 1 && n_rows <= 3 * min_split_rows ? 1u : 0u;
-    if (*single) {
-        *split_len = (n_rows + 15) / 16 * 16;
-        *n_splits = 1;
-        *heads_per_wg = 1;
-        return;
-    }
     uint32_t len = (n_rows + want - 1) / want;
     if (len < min_split_rows) len = min_split_rows;
     len = (len + batch_rows - 1) / batch_rows * batch_rows;
-    *split_len = len;
-    *n_splits = n_rows == 0 ? 1 : (n_rows + len - 1) / len;
-    *heads_per_wg = h;
+    a.split_len = len;
+    a.n_splits = n_rows == 0 ? 1 : (n_rows + len - 1) / len;
+    a.heads_per_wg = h;
+    // The merge pass costs a launch, so at the shortest contexts one workgroup takes a
+    // KV head's whole context and stores the output itself (no_merge): the 4-wave
+    // layout for a plain decode of one split, else the single layout's 8 waves, while
+    // no SIMD has more than 5 of the 16-row batches (one of its two waves a third
+    // one; a batch costs a wave about 1 us). Us in graph replays, 8 KV heads, at 100 /
+    // 200 / 320 / 336 rows: fused step single 5.4 / 5.6 / 6.3 / 7.2, split + merge
+    // 6.8 / 6.7 / 6.8 / 6.7; plain 4 waves 3.5, single 4.2 / 4.7 / 5.4 / 6.2, split +
+    // merge from 129 rows on 5.8 / 5.9 / 5.9. Not where a workgroup's output could
+    // land in what another still reads: the merge stores it after all have read.
+    const bool one_split = !fused && a.n_splits == 1;
+    a.single = may_one_launch && h == 1 && !one_split && 2ull * n_rows <= 5 * min_split_rows ? 1u : 0u;
+    a.no_merge = a.single || (may_one_launch && one_split) ? 1u : 0u;
+    if (a.single) {
+        a.split_len = (n_rows + 15) / 16 * 16;
+        a.n_splits = 1;
+    }
 }
 
 uint32_t decode_max_splits() { return kMaxSplits; }
@@ -706,14 +717,14 @@ static void launch_merge(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s)
 
 hipError_t launch_decode(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s) {
     launch_split<false>(a, n_kv_head, s);
-    if (!a.single)
+    if (!a.no_merge)
         launch_merge<false>(a, n_kv_head, s);
     return hipGetLastError();
 }
 
 hipError_t launch_decode_step(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s) {
     launch_split<true>(a, n_kv_head, s);
-    if (!a.single)
+    if (!a.no_merge)
         launch_merge<true>(a, n_kv_head, s);
     return hipGetLastError();
 }

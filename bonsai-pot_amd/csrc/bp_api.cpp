@@ -159,15 +159,15 @@ bool overlap(const uint16_t* a, uint64_t na, const uint16_t* b, uint64_t nb) {
     return x < y + 2 * nb && y < x + 2 * na;
 }
 
-// The single decode layout reads and writes act in one launch, a workgroup per KV
-// head: out may be q itself (each workgroup reads its own heads before it stores
+// Without a merge pass one launch reads and writes act, a workgroup per KV head (or
+// four): out may be q itself (each workgroup reads its own heads before it stores
 // them), but not lie across other heads' q.
-bool decode_may_single(const uint16_t* q, const uint16_t* out, uint32_t q_dim) {
+bool decode_may_one_launch(const uint16_t* q, const uint16_t* out, uint32_t q_dim) {
     return q == out || !overlap(q, q_dim, out, q_dim);
 }
 
 bp::DecodeArgs decode_args(const bp_model* m, void* act, uint32_t q_off, uint32_t out_off, uint32_t il,
-                           uint32_t n_rows, bool may_single) {
+                           uint32_t n_rows, bool fused, bool may_one_launch) {
     bp::DecodeArgs a{};
     a.q = static_cast<const uint16_t*>(act) + q_off;
     a.out = static_cast<uint16_t*>(act) + out_off;
@@ -176,9 +176,8 @@ bp::DecodeArgs decode_args(const bp_model* m, void* act, uint32_t q_off, uint32_
     a.partials = m->partials;
     a.kv_dim = m->kv_dim;
     a.n_rows = n_rows;
-    bp::decode_plan(n_rows, m->cfg.n_kv_head, m->cu_count, m->decode_min_split_rows, m->decode_wide_min_rows,
-                    may_single && decode_may_single(a.q, a.out, m->q_dim), &a.split_len, &a.n_splits,
-                    &a.heads_per_wg, &a.single);
+    bp::decode_plan(a, m->cfg.n_kv_head, m->cu_count, m->decode_min_split_rows, m->decode_wide_min_rows, fused,
+                    may_one_launch && decode_may_one_launch(a.q, a.out, m->q_dim));
     a.scale = 1.0f / std::sqrt(static_cast<float>(m->cfg.head_dim));   // src/forward.rs:838
     return a;
 }
@@ -477,7 +476,7 @@ bp_status bp_dispatch_attention_decode(bp_model* m, void* act, uint32_t q_off, u
                     m->max_seq);
     if ((q_off & 7u) || (out_off & 3u))
         return fail(BP_ERR_INVALID_ARG, "q_off must be a multiple of 8 and out_off of 4 (aligned f16 rows)");
-    bp::DecodeArgs a = decode_args(m, act, q_off, out_off, layer_il, pos + 1, true);   // src/forward.rs:822
+    bp::DecodeArgs a = decode_args(m, act, q_off, out_off, layer_il, pos + 1, false, true);   // src/forward.rs:822
     if (static_cast<uint64_t>(a.n_splits) * m->cfg.n_head * bp::decode_partial_stride() > m->partials_floats)
         return fail(BP_ERR_CONFIG, "internal: partials scratch too small for %u splits", a.n_splits);
     return hip_check(m, bp::launch_decode(a, m->cfg.n_kv_head, m->stream), "attention_decode launch");
@@ -504,10 +503,11 @@ bp_status bp_dispatch_attention_decode_step(bp_model* m, void* act, const void* 
     const uint16_t* const w = static_cast<const uint16_t*>(w_norms);
     const struct { const uint16_t* at; uint32_t n; } reads[] = {{x + k_cur_off, m->kv_dim}, {x + v_cur_off, m->kv_dim},
         {w + w_q_norm_off, m->cfg.head_dim}, {w + w_k_norm_off, m->cfg.head_dim}};
-    bool may_single = true;
+    bool may_one_launch = true;
     for (const auto& r : reads)
-        may_single = may_single && !overlap(x + out_off, m->q_dim, r.at, r.n) && !overlap(x + q_off, m->q_dim, r.at, r.n);
-    bp::DecodeArgs a = decode_args(m, act, q_off, out_off, layer_il, pos, may_single);
+        may_one_launch = may_one_launch && !overlap(x + out_off, m->q_dim, r.at, r.n) &&
+                         !overlap(x + q_off, m->q_dim, r.at, r.n);
+    bp::DecodeArgs a = decode_args(m, act, q_off, out_off, layer_il, pos, true, may_one_launch);
     a.q_act = x + q_off;
     a.q_norm = m->q_norm;
     a.k_cur = x + k_cur_off;
@@ -998,9 +998,8 @@ bp_status bp_attention_decode_noalloc(const bp_config* cfg, void* kv_k, void* kv
     a.partials = d->ptr;
     a.kv_dim = kv_dim;
     a.n_rows = pos + 1;   // src/forward.rs:822
-    bp::decode_plan(a.n_rows, cfg->n_kv_head, d->cu_count, bp::kDecodeMinSplitRows, bp::kDecodeWideMinRows,
-                    decode_may_single(a.q, a.out, cfg->n_head * cfg->head_dim), &a.split_len, &a.n_splits,
-                    &a.heads_per_wg, &a.single);
+    bp::decode_plan(a, cfg->n_kv_head, d->cu_count, bp::kDecodeMinSplitRows, bp::kDecodeWideMinRows, false,
+                    decode_may_one_launch(a.q, a.out, cfg->n_head * cfg->head_dim));
     a.scale = 1.0f / std::sqrt(static_cast<float>(cfg->head_dim));   // src/forward.rs:838
     if (static_cast<uint64_t>(a.n_splits) * cfg->n_head * bp::decode_partial_stride() > kNoAllocScratchFloats)
         return fail(BP_ERR_CONFIG, "noalloc decode: %u query heads x %u splits exceed the %llu-float scratch",

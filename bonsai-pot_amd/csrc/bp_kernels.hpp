@@ -78,7 +78,8 @@ struct DecodeArgs {
     uint64_t w_q_off, w_k_off;
     uint32_t pos;
     float eps;
-    uint32_t single;          // 1: the single layout, one launch (n_splits = heads_per_wg = 1)
+    uint32_t single;          // 1: the single layout (n_splits = heads_per_wg = 1)
+    uint32_t no_merge;        // 1: the one split's workgroups store the output, no merge pass
 };
 
 struct PrefillArgs {
@@ -206,19 +207,19 @@ hipError_t launch_q_norm_rope(const QNormRopeArgs& a, uint32_t n_head, uint32_t 
                               hipStream_t s);
 hipError_t launch_kv_writeback(const KvWritebackArgs& a, uint32_t n_kv_head, uint32_t m_tokens,
                                hipStream_t s);
-// Split-K plan of a decode over n_rows rows (1 <= n_splits <= decode_max_splits())
-// and the split pass's layout (heads_per_wg = 4 from wide_min_rows rows on), or
-// where may_single the single layout at the shortest contexts.
-void decode_plan(uint32_t n_rows, uint32_t n_kv_head, int cu_count, uint32_t min_split_rows,
-                 uint32_t wide_min_rows, bool may_single, uint32_t* split_len, uint32_t* n_splits,
-                 uint32_t* heads_per_wg, uint32_t* single);
+// Split-K plan of a decode over a.n_rows rows: the split pass's layout (single, or
+// 1 or 4 KV heads per workgroup, 4 from wide_min_rows rows on), its splits
+// (1 <= n_splits <= decode_max_splits()) and, where may_one_launch, whether they
+// store the output without a merge pass.
+void decode_plan(DecodeArgs& a, uint32_t n_kv_head, int cu_count, uint32_t min_split_rows, uint32_t wide_min_rows,
+                 bool fused, bool may_one_launch);
 uint32_t decode_max_splits();
 uint32_t decode_partial_stride();   // floats per (head, split) partial
-// Plain decode (q already normalized, cache row already written): one launch in
-// the single layout, else split pass + merge pass.
+// Plain decode (q already normalized, cache row already written): split pass,
+// and merge pass unless no_merge.
 hipError_t launch_decode(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s);
-// Fused decode step: split pass (with q norm + row writeback) + merge pass, or
-// the single layout's one launch.
+// Fused decode step: split pass (with q norm + row writeback), and merge pass
+// unless no_merge (the single layout).
 hipError_t launch_decode_step(const DecodeArgs& a, uint32_t n_kv_head, hipStream_t s);
 hipError_t launch_prefill(const PrefillArgs& a, uint32_t n_kv_head, hipStream_t s);
 // Whether the launches of launch_prefill (step = false) or launch_prefill_step

@@ -140,6 +140,25 @@ def h2d(ptr: int, host: np.ndarray) -> None:
     assert rc == 0, f"hipMemcpy H2D failed: {rc}"
 
 
+def launches_of(model, body) -> int:
+    """Kernel launches that body() makes on model's stream, counted as the nodes of
+    a captured graph; nothing runs."""
+    import torch
+    hip, side = hip_runtime(), torch.cuda.Stream()
+    graph, n = ctypes.c_void_p(), ctypes.c_size_t()
+    torch.cuda.synchronize()
+    model.set_stream(side.cuda_stream)
+    assert hip.hipStreamBeginCapture(ctypes.c_void_p(side.cuda_stream), 2) == 0   # relaxed mode
+    try:
+        body()
+    finally:
+        assert hip.hipStreamEndCapture(ctypes.c_void_p(side.cuda_stream), ctypes.byref(graph)) == 0
+        model.set_stream(torch.cuda.current_stream().cuda_stream)
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    assert hip.hipGraphDestroy(graph) == 0
+    return n.value
+
+
 class DeviceScenario:
     """Uploads a Scenario's act / w_norms into torch device memory and creates a
     Model whose KV cache starts as the scenario's (usually zero) KV bytes."""

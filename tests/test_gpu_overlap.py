@@ -4,40 +4,19 @@ may lie over k_cur / v_cur (dead once the row is written) and over q. Where a
 workgroup of the one-launch layout could store into what another still reads,
 the step takes two launches; the launches are counted in a captured graph.
 """
-import ctypes
 import sys
 
 import numpy as np
 import pytest
 
-from bonsai_pot_amd import layout, lib
-from helpers import DeviceScenario, Scenario, assert_attn_close
+from bonsai_pot_amd import layout
+from helpers import DeviceScenario, Scenario, assert_attn_close, launches_of
 
 pytestmark = pytest.mark.gpu
-
-_vp = ctypes.c_void_p
-
 
 def _say(*a):
     print(*a, flush=True)
     sys.stdout.flush()
-
-
-def _nodes(model, body):
-    """Nodes that body() records on model's stream; nothing runs."""
-    import torch
-    side, graph, n = torch.cuda.Stream(), _vp(), ctypes.c_size_t()
-    torch.cuda.synchronize()
-    model.set_stream(side.cuda_stream)
-    assert lib.hipStreamBeginCapture(_vp(side.cuda_stream), 2) == 0   # relaxed
-    try:
-        body()
-    finally:
-        assert lib.hipStreamEndCapture(_vp(side.cuda_stream), ctypes.byref(graph)) == 0
-        model.set_stream(torch.cuda.current_stream().cuda_stream)
-    assert lib.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
-    assert lib.hipGraphDestroy(graph) == 0
-    return n.value
 
 
 def _scenario(pos, n_kv, seed):
@@ -51,20 +30,20 @@ def _scenario(pos, n_kv, seed):
 
 
 # act is q | k | v | out; out moved to the named place (element offsets), and the
-# launches of the step at up to 384 rows
+# launches of the step at up to 320 rows
 PLACES = {"apart": (lambda sc: sc.out_off, 1), "q": (lambda sc: sc.q_off, 1), "k": (lambda sc: sc.k_off, 2),
           "v": (lambda sc: sc.v_off, 2), "end of v": (lambda sc: sc.v_off + sc.cfg.kv_dim - 4, 2)}
 
 
 @pytest.mark.parametrize("place", sorted(PLACES))
-@pytest.mark.parametrize("pos,n_kv", [(0, 8), (100, 8), (300, 12), (384, 1), (385, 8)])
+@pytest.mark.parametrize("pos,n_kv", [(0, 8), (100, 8), (300, 12), (320, 1), (321, 8)])
 def test_decode_step_out_over_inputs(cuda, place, pos, n_kv):
     _say(f"[overlap] decode step out over {place} pos={pos} n_kv_head={n_kv}")
     at, launches = PLACES[place]
     sc = _scenario(pos, n_kv, seed=1500 + pos)
     sc.out_off = at(sc)
     dev = DeviceScenario(sc, upload_kv=True)
-    assert _nodes(dev.model, lambda: dev.decode_step(1, pos)) == (launches if pos <= 384 else 2)
+    assert launches_of(dev.model, lambda: dev.decode_step(1, pos)) == (launches if pos <= 320 else 2)
     dev.decode_step(1, pos)
     sc.oracle_q_norm_rope(pos)
     sc.oracle_writeback(1, pos)
@@ -78,14 +57,14 @@ def test_decode_step_out_over_inputs(cuda, place, pos, n_kv):
 
 
 @pytest.mark.parametrize("shift,launches", [(0, 1), (512, 2), (4, 2), (4096, 1)])
-@pytest.mark.parametrize("pos", [100, 300])
+@pytest.mark.parametrize("pos", [100, 127, 128, 300])
 def test_decode_out_over_q(cuda, shift, launches, pos):
     """The plain decode with out on q itself, across other heads' q, behind q."""
     _say(f"[overlap] decode out over q + {shift} pos={pos}")
     sc = _scenario(pos + 1, 8, seed=1600 + pos)
     sc.out_off = sc.q_off + shift
     dev = DeviceScenario(sc, upload_kv=True)
-    assert _nodes(dev.model, lambda: dev.decode(1, pos)) == launches
+    assert launches_of(dev.model, lambda: dev.decode(1, pos)) == launches
     dev.decode(1, pos)
     _, want = sc.oracle_decode(1, pos)
     assert_attn_close(dev.out_f32(1)[0], want, f"decode, out over q + {shift}, pos={pos}")
@@ -110,7 +89,7 @@ def test_prefill_step_out_over_q(cuda, m, pos, shift, launches):
     def step():
         dev.model.dispatch_attention_prefill_step(dev.act.data_ptr(), dev.w.data_ptr(), sc.q_off, sc.k_off, sc.v_off,
                                                   sc.out_off, sc.w_q_off, sc.w_k_off, 1, pos, m)
-    assert _nodes(dev.model, step) == launches
+    assert launches_of(dev.model, step) == launches
     step()
     sc.oracle_q_norm_rope(pos)
     sc.oracle_writeback(1, pos)

@@ -10,7 +10,7 @@ import pytest
 
 import oracle as orc
 from bonsai_pot_amd import layout
-from helpers import DeviceScenario, Scenario, assert_attn_close, write_outlier_rows
+from helpers import DeviceScenario, Scenario, assert_attn_close, launches_of, write_outlier_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -390,18 +390,23 @@ def test_prefill_key_split(cuda, monkeypatch, m, pos_base, ksplit):
     assert_attn_close(dev.out_f32(), want, f"prefill key split m={m} pos_base={pos_base} ksplit={ksplit}")
 
 
-# The single layout (one workgroup per KV head, up to 3 x 128 rows) at the edges of
-# its batches and where the split layout takes over; rows of a second model without
-# it (BP_DECODE_MIN_SPLIT_ROWS 32: splits of 64 rows) agree within the same bar.
-@pytest.mark.parametrize("pos", [0, 1, 15, 16, 17, 127, 128, 129, 255, 383, 384, 385])
+# One launch up to 5/2 of the minimum split (320 rows; the fused step in the single
+# layout, the plain decode in the 4-wave layout while it is one split of 128 rows),
+# at the edges of its batches and where split + merge takes over. A second model
+# (BP_DECODE_MIN_SPLIT_ROWS 32: one launch up to 80 rows, splits of 64 rows beyond)
+# runs the other layout over most of the same rows.
+@pytest.mark.parametrize("pos", [0, 1, 15, 16, 17, 80, 81, 97, 127, 128, 129, 255, 319, 320, 321, 383, 384, 385])
 def test_decode_single_layout(cuda, monkeypatch, pos):
     _say(f"[decode single] pos={pos}")
     cfg = layout.Config(n_layer=2)
     for min_rows in ("128", "32"):
+        one_launch = 5 * int(min_rows) // 2
         monkeypatch.setenv("BP_DECODE_MIN_SPLIT_ROWS", min_rows)
         sc = Scenario(cfg, max_seq=pos + 8, m_tokens=1, seed=700 + pos, w_std=0.2)
         _prefill_cache(sc, 1, pos, seed=800 + pos)
         dev = DeviceScenario(sc, upload_kv=True)
+        assert launches_of(dev.model, lambda: dev.decode_step(1, pos)) == (1 if pos <= one_launch else 2)
+        assert launches_of(dev.model, lambda: dev.decode(1, pos)) == (1 if pos + 1 <= one_launch else 2)
         dev.decode_step(1, pos)
         sc.oracle_q_norm_rope(pos)
         sc.oracle_writeback(1, pos)
