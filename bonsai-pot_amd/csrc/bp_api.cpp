@@ -568,18 +568,33 @@ static bp_status prefill_args(bp_model* m, void* act, uint32_t q_off, uint32_t o
             }
             return ns > 1;
         };
-        // Kernel (us of the fused step below; BP_PREFILL_HEADS_PER_WAVE,
-        // BP_PREFILL_WG_WAVES and BP_PREFILL_KSPLIT force one):
-        //  * prefill_kernel, the one-head 16x16 kernel with 4 waves, for at most 5
-        //    key chunks, and 8 while at most a quarter of the rows lie before the
-        //    chunk (half the scores of its tile pairs are masked): 64 / 256 / 448
-        //    tokens from an empty cache 12.1 / 16.4 / 19.3, prefill32_kernel 14.5 /
-        //    17.0 / 20.5; but 200 on 250 rows 21.6 and 20.1;
-        //  * prefill_split_kernel (reads the cache's own rows, no image) for few
-        //    tiles over a long cache, from 32 chunks per tile on, where writing the
+        // Kernel (us of the fused step in graph replays at 8 KV heads unless it says
+        // otherwise; BP_PREFILL_HEADS_PER_WAVE, BP_PREFILL_WG_WAVES and
+        // BP_PREFILL_KSPLIT force one):
+        //  * prefill_split_kernel (reads the cache's own rows, no image) for few tiles
+        //    over a long cache. One tile: from 6 chunks on (16 tokens on 500 / 1000 rows
+        //    16.0 / 16.0, prefill32_kernel 20.1 / 20.9), or 10 where the partials of
+        //    that many heads cost more (32 tokens of 16 KV heads on 300 rows 19.5,
+        //    prefill_kernel 16.4). More: from 32 chunks per tile on, where writing the
         //    image costs more than converting in the workgroups (64 tokens on 16384
-        //    rows 54, prefill32_kernel 69; 128 on 8192 52 and 51), and for a single
-        //    tile (16 on 500 / 1000 rows 16.0 / 16.0, prefill32_kernel 20.1 / 20.9);
+        //    rows 54, prefill32_kernel 69; 128 on 8192 52 and 51), 24 and 8 with more KV
+        //    heads (16: 100 on 8000 68.7 and 73.9; 32: 64 on 3000 45.8 and 52.3); and two
+        //    tiles with little in the second from 9 or 12 (33 on 700 20.1 and 21.5; 4 KV
+        //    heads, 48 on 2000 22.6 and 24.2); one or two KV heads, whose 32x32 grid
+        //    stays small, over 10 to 20 chunks (1: 64 on 800 19.5 and 22.8).
+        //  * prefill_kernel, the one-head 16x16 kernel with 4 waves, for few chunks: 5, or
+        //    more while the light tiles of its zig-zag pairs see few of them (64 / 256 /
+        //    448 tokens from an empty cache 12.1 / 16.4 / 19.3, prefill32_kernel 14.5 /
+        //    17.0 / 20.5; 384 on 30 rows 19.0 and 20.5, 4 KV heads and 1024 on 10 28.5
+        //    and 30.0; but 200 on 250 21.6 and 20.3), or
+        //    while its 16-token units leave the second half of two or three tiles out
+        //    (33 on 400 19.0 and 19.8). Not causal: 5 chunks, 7 for 33 to 48 tokens,
+        //    and one tile (attention alone: 16 tokens on 500 / 8000 rows 15.0 / 110,
+        //    prefill32_kernel 18.1 / 122; 32 on 1500 36.0 and 34.8);
+        //  * with 8 waves where 4 do not fit the CUs, for a single chunk not causal
+        //    (1024 tokens on 64 rows 14.4, prefill32_kernel 15.3; on 128 16.0 and 16.2),
+        //    or an uneven number of heads (below) near an empty cache (12: 384 tokens on
+        //    30 rows 22.6 and 24.2; on 64 23.5 and 23.1);
         //  * else prefill32_kernel.
         // With out across q (neither apart nor q itself) the other two would store into
         // what another workgroup still reads; the split kernel stores in its merge, so
@@ -587,34 +602,55 @@ static bp_status prefill_args(bp_model* m, void* act, uint32_t q_off, uint32_t o
         a.heads_per_wave = m->prefill_hpw != 0 ? m->prefill_hpw : 2u;
         const uint64_t elems = static_cast<uint64_t>(m_tokens) * m->q_dim;
         const bool across = a.q != a.out && overlap(a.q, elems, a.out, elems);
-        const uint64_t from = across ? 4ull * a.n_tiles : a.n_tiles == 1 ? 6 : 32ull * a.n_tiles;
+        // More than 8 KV heads that 8 does not divide spread unevenly over the 8 XCDs, which
+        // costs prefill32_kernel's few large workgroups more: 12 heads, 128 tokens on 200
+        // rows 19.8 (prefill_kernel) and 21.1, 48 on 800 23.9 (split kernel) and 25.6.
+        const bool uneven = n_kv > 8 && n_kv % 8 != 0;
+        const bool light = a.n_tiles == 1 && m_tokens * n_kv <= 320;   // partials of many splits stay few
+        uint64_t from = (n_kv >= 24 ? 8ull : n_kv >= 16 ? 24ull : 32ull) * a.n_tiles;
+        if (a.n_tiles == 1) from = light ? 6 : 10;
+        else if (m_tokens <= 40) from = std::min<uint64_t>(from, n_kv <= 12 ? 9 : 12);
+        else if (m_tokens <= 48 && (n_kv <= 4 || uneven)) from = 12;
+        if (n_kv <= 2 && a.n_tiles >= 2 && a.n_tiles <= 4 && chunks <= 20) from = 10;
+        if (across) from = 4ull * a.n_tiles;
         if (m->prefill_hpw != 2 && is_prefill && small && m->prefill_waves != 8 &&
             (m->prefill_ksplit != 0 || chunks >= from)) {
-            // one 8-wave workgroup per (KV head, key split, tile pair): enough splits
-            // to give every CU a workgroup, at least 2 chunks each (a single tile: 1,
-            // up to 16 splits; 16 tokens on 1000 rows: 8 splits 16.9, 16 16.0)
+            // one 8-wave workgroup per (KV head, key split, tile pair): enough splits to
+            // give every CU a workgroup, at least 2 chunks each (a single light tile over
+            // up to 12 or 20 chunks: 1, up to 16 splits; 16 tokens on 1000 rows: 8 splits
+            // 16.9, 16 16.0; 16 KV heads, 20 on 1000: 19.5 and 21.1)
             const uint32_t wgs = pairs * n_kv;
             uint32_t most = chunks / 2;
-            if (a.n_tiles == 1) most = std::max(most, std::min(chunks, 16u));
+            if (light && chunks <= (m_tokens * n_kv <= 192 ? 20u : 12u)) most = std::max(most, std::min(chunks, 16u));
             if (split_keys(m->prefill_ksplit != 0 ? m->prefill_ksplit : std::min<uint32_t>((cus + wgs - 1) / wgs, most))) {
                 a.direct = 1;
                 a.heads_per_wave = 1;
             }
         }
-        const bool few = chunks <= 5 || (chunks <= 8 && 4 * static_cast<uint64_t>(m_tokens) >= 3 * rows);
-        if (m->prefill_hpw == 0 && !a.direct && small && (few || m->prefill_waves != 0)) a.heads_per_wave = 1;
+        const uint64_t first = (static_cast<uint64_t>(pos) + 95) / 64;   // the first tile's key chunks
+        bool few = chunks <= (is_prefill && uneven ? 7u : 5u);
+        if (is_prefill)
+            few = few || 5 * first + chunks <= 22 || (a.n_tiles == 1 && !light) ||
+                  (a.n_tiles <= 3 && chunks <= 7 && (m_tokens - 1) % 32 < 16);
+        else
+            few = few || (a.n_tiles == 1 && (m_tokens <= 16 || chunks <= (n_kv <= 4 ? 32u : 16u))) ||
+                  (a.n_tiles == 2 && chunks <= 7 && m_tokens <= 48);
+        const bool eight = 2 * pairs * n_kv <= cus &&
+                           (is_prefill ? uneven && first == 1 && chunks <= 9 : chunks == 1);
+        if (m->prefill_hpw == 0 && !a.direct && ((small && (few || m->prefill_waves != 0)) || eight)) a.heads_per_wave = 1;
         a.wg_waves = 8;
         if (a.heads_per_wave == 1) a.wg_waves = m->prefill_waves != 0 ? m->prefill_waves : (small ? 4u : 8u);
         // prefill32_kernel: one tile per workgroup while all tiles fit the CUs (512
         // tokens on 2048 rows 48.6, as pairs 74.6; 777 on 1501 49.8 and 67.6), or
         // while the tiles beyond them are so light that two take less than the
         // heaviest one (1025 tokens from an empty cache 31.1 and 38.0); else zig-zag
-        // pairs (2048: 65.8 and 64.2; 1200 on 3000: 122 and 116).
+        // pairs (2048: 65.8 and 64.2; 1200 on 3000: 122 and 116; 12 heads, 1100 from an
+        // empty cache 46.0 and 44.0).
         const uint32_t wgs = a.n_tiles * n_kv;
         a.tiles_per_wg = 2;
         if (wgs <= cus) {
             a.tiles_per_wg = 1;
-        } else if (wgs <= 2 * cus && is_prefill) {
+        } else if (wgs <= 2 * cus && is_prefill && !uneven) {
             const uint32_t next = a.n_tiles - 1 - cus / n_kv;   // the heaviest tile beyond the first round
             a.tiles_per_wg = 2 * ((static_cast<uint64_t>(pos) + 32 * next + 95) / 64) < chunks ? 1 : 2;
         }

@@ -52,9 +52,10 @@ def test_writeback_and_q_norm_rope(cuda, kv):
 
 
 @pytest.mark.parametrize("kv", KV_HEADS)
-@pytest.mark.parametrize("pos", [300, 9000])
+@pytest.mark.parametrize("pos", [300, 500, 9000])
 def test_decode_step(cuda, kv, pos):
-    """The fused step; at 9000 rows the wide layout runs when n_kv_head % 4 == 0."""
+    """The fused step: the single layout at 300 rows, narrow splits at 500, and at
+    9000 the wide layout when n_kv_head % 4 == 0."""
     _say(f"[heads] decode step n_kv_head={kv} pos={pos}")
     cfg = _cfg(kv)
     sc = Scenario(cfg, max_seq=pos + 4, m_tokens=1, seed=20 + kv + pos)
@@ -128,3 +129,25 @@ def test_prefill_key_split(cuda, monkeypatch, kv):
     dev.attention(0, pos, is_prefill=True)
     want = sc.oracle_attention(0, pos, is_prefill=True)
     assert_attn_close(dev.out_f32(), want, f"prefill key split n_kv_head={kv}")
+
+
+# Default choices that depend on the head count: the split kernel (a few tiles over 10
+# to 20 chunks at 1 or 2 heads, from 24 or 8 chunks per tile at 16 or 32), the 16x16
+# kernel with 4 waves and 8 (12 heads near an empty cache), prefill32_kernel with one
+# tile per workgroup, with a key split, with light tiles beyond the CUs (4) and on
+# pairs with an odd number of tiles and a ragged last one (12).
+@pytest.mark.parametrize("kv,m,pos", [(1, 64, 800), (1, 64, 1300), (2, 100, 700), (2, 300, 900), (4, 48, 800), (4, 64, 1000), (4, 700, 900),
+                                      (4, 2100, 100), (12, 24, 500), (12, 48, 800), (12, 64, 1000), (12, 128, 200), (12, 384, 30),
+                                      (12, 260, 900), (12, 900, 300), (12, 740, 40), (16, 24, 300), (16, 64, 3040), (16, 64, 2900),
+                                      (16, 500, 200), (32, 16, 700), (32, 33, 700), (32, 100, 2000), (32, 200, 600)])
+def test_prefill_default_choices(cuda, kv, m, pos):
+    _say(f"[heads] prefill choices n_kv_head={kv} m={m} pos={pos}")
+    sc = Scenario(_cfg(kv), max_seq=pos + m, m_tokens=m, seed=100 + kv + m)
+    _prefill_cache(sc, 0, pos, seed=110 + kv)
+    sc.oracle_q_norm_rope(pos)
+    sc.oracle_writeback(0, pos)
+    dev = DeviceScenario(sc, upload_kv=True)
+    dev.attention(0, pos, is_prefill=True)
+    tokens = np.unique(np.concatenate([np.arange(0, m, 37), [t for t in (1, 15, 16, 31, 32, m - 2, m - 1) if 0 <= t < m]])).astype(int)
+    want = sc.oracle_attention(0, pos, is_prefill=True, tokens=tokens)
+    assert_attn_close(dev.out_f32()[tokens], want, f"prefill n_kv_head={kv} m={m} pos={pos}")

@@ -165,9 +165,9 @@ def test_decode_ctx32k_with_outlier_rows(cuda):
                                         (130, 1000), (33, 31), (200, 900)])
 @pytest.mark.parametrize("hpw", ["1", "1w4", "2"])
 def test_prefill_vs_oracle(cuda, monkeypatch, m, pos_base, hpw):
-    """Every prefill_kernel layout (1 query head per wave in 8- or 4-wave
-    workgroups, or 2 per wave; by default the grid size picks one), forced
-    through BP_PREFILL_HEADS_PER_WAVE and BP_PREFILL_WG_WAVES. (200, 900)
+    """Every layout over the image (the 16x16 kernel in 8- or 4-wave workgroups,
+    prefill32_kernel; by default the shape picks one), forced through
+    BP_PREFILL_HEADS_PER_WAVE and BP_PREFILL_WG_WAVES. (200, 900)
     gives second-half units whose first chunk lies wholly past some tokens'
     last row (all scores masked while the running max is still unset)."""
     monkeypatch.setenv("BP_PREFILL_HEADS_PER_WAVE", hpw[0])
@@ -184,17 +184,22 @@ def test_prefill_vs_oracle(cuda, monkeypatch, m, pos_base, hpw):
     assert_attn_close(dev.out_f32(), want, f"prefill m={m} pos_base={pos_base}")
 
 
-def test_attention_non_causal_multi_token(cuda):
-    """is_prefill = 0: every token sees rows [0, pos) (attention.wgsl:263)."""
-    _say("[prefill] non-causal")
+@pytest.mark.parametrize("m,pos", [(40, 250), (16, 700), (17, 1024), (17, 1025), (48, 400), (49, 400), (100, 600), (600, 60), (600, 65),
+                                   (1030, 640)])
+def test_attention_non_causal_multi_token(cuda, m, pos):
+    """is_prefill = 0: every token sees rows [0, pos) (attention.wgsl:263). The 16x16
+    kernel with 4 waves (few chunks, or a single tile) and 8 (600 on 60),
+    prefill32_kernel by tiles and by pairs (1030: 33 tiles)."""
+    _say(f"[prefill] non-causal m={m} pos={pos}")
     cfg = layout.Config(n_layer=1)
-    sc = Scenario(cfg, max_seq=300, m_tokens=40, seed=9)
-    _prefill_cache(sc, 0, 250, seed=10)
-    sc.oracle_q_norm_rope(250)
+    sc = Scenario(cfg, max_seq=pos + m + 10, m_tokens=m, seed=9 + m)
+    _prefill_cache(sc, 0, pos, seed=10 + m)
+    sc.oracle_q_norm_rope(pos)
     dev = DeviceScenario(sc, upload_kv=True)
-    dev.attention(0, 250, is_prefill=False)
-    want = sc.oracle_attention(0, 250, is_prefill=False)
-    assert_attn_close(dev.out_f32(), want, "non-causal")
+    dev.attention(0, pos, is_prefill=False)
+    tokens = np.arange(m) if m <= 64 else np.unique(np.concatenate([np.arange(0, m, 29), [31, 32, m - 2, m - 1]]))
+    want = sc.oracle_attention(0, pos, is_prefill=False, tokens=tokens)
+    assert_attn_close(dev.out_f32()[tokens], want, f"non-causal m={m} pos={pos}")
 
 
 @pytest.mark.parametrize("m,pos_base", [(2048, 0), (2048, 2048), (64, 16384)])
@@ -224,8 +229,8 @@ def test_prefill_full_size_sampled_rows(cuda, m, pos_base):
 @pytest.mark.parametrize("m,pos_base", [(100, 30000), (1000, 8000), (2048, 6000)])
 def test_prefill_long_cache_sampled_rows(cuda, m, pos_base):
     """Chunks over long caches in each layout the library picks by default:
-    100 tokens on 30000 rows (the key split), 1000 on 8000 (the one-head
-    8-wave kernel over the image) and 2048 on 6000 (prefill32_kernel); the
+    100 tokens on 30000 rows (the key split), 1000 on 8000 (prefill32_kernel,
+    one tile per workgroup) and 2048 on 6000 (prefill32_kernel on pairs); the
     oracle checks sampled tokens of every 64-token tile, first and last
     included."""
     _say(f"[prefill-long] m={m} pos_base={pos_base}")
@@ -420,14 +425,19 @@ def test_decode_single_layout(cuda, monkeypatch, pos):
         assert_attn_close(dev.out_f32(1)[0], want, f"decode pos={pos}")
 
 
-# The choices between the prefill kernels at their edges: 5 and 6 key chunks,
-# and 8 and 9 from an empty cache (16x16 / 32x32 kernel; a single tile: the split kernel), one tile per
-# workgroup with 1, 2, 4 and 8 key splits (49 chunks in 8 splits of 7: one
-# has none), as many tiles as CUs / KV heads (32) and one more (light
-# tiles beyond the first round, or pairs), 32 chunks per tile (the split kernel).
-@pytest.mark.parametrize("m,pos_base", [(129, 191), (129, 192), (512, 0), (513, 0), (32, 288), (32, 289), (31, 700), (33, 351), (64, 1000),
-                                        (64, 3072), (128, 3008), (65, 1300), (256, 1600), (255, 3000), (400, 2560), (512, 3300), (512, 100),
-                                        (1024, 33), (1025, 0), (1025, 64), (1056, 700), (64, 4032), (64, 4031)])
+# The choices between the prefill kernels at their edges (8 KV heads): the 16x16
+# kernel at 5 chunks, at up to 17 from an empty cache, and at 6 and 7 where the last
+# tile is half empty, next to prefill32_kernel; a single tile (5, 6, 12 and 13, 20 and
+# 21 chunks) and two tiles of 33 to 40 tokens (8 and 9) on the split kernel; one tile
+# per workgroup with 1, 2, 4 and 8 key splits (49 chunks in 8 splits of 7: one has
+# none), as many tiles as CUs / KV heads (32) and one more, light (one tile per
+# workgroup) or not (zig-zag pairs: an odd number of tiles and a ragged last one, also
+# beyond 2 x CUs tiles); 32 chunks per tile (the split kernel).
+@pytest.mark.parametrize("m,pos_base", [(129, 191), (129, 192), (512, 0), (513, 0), (544, 30), (32, 288), (32, 289), (31, 700), (24, 740),
+                                        (24, 760), (8, 1272), (8, 1273), (33, 351), (65, 300), (65, 383), (64, 300), (33, 479), (40, 472),
+                                        (40, 473), (41, 560), (64, 1000), (64, 3072), (128, 3008), (65, 1300), (256, 1600), (255, 3000),
+                                        (400, 2560), (512, 3300), (512, 100), (1024, 33), (1025, 0), (1025, 64), (1056, 700), (1050, 1500),
+                                        (2115, 0), (64, 4032), (64, 4031)])
 def test_prefill_default_choices(cuda, m, pos_base):
     _say(f"[prefill choices] m={m} pos_base={pos_base}")
     cfg = layout.Config(n_layer=1)
