@@ -11,24 +11,27 @@
 //    the exact integer sum of +-q over the 32 elements (bit e of the row's
 //    block selects +q[e]); then f16(acc), or f16(f32(y) + acc) to accumulate.
 //
-// Matmul on the i8 matrix cores, weight rows as A and tokens as B of 16 x 16
-// MFMAs, so that a lane holds four consecutive rows of one token. What bounds
-// it is issue: per (output, 32-block) the order of the sums leaves one
-// subtraction, one product and one addition in f32 (the scale a_d * w_d comes
-// from the matrix core, sumi needs no conversion; see below), and a wave alone
-// on its SIMD issues one instruction per six cycles (two waves: three cycles;
-// four: 2.4), while the MFMAs add their own time. The kernels differ in how
-// much of the machine a shape fills:
+// Matmul on the i8 matrix cores, one v_mfma_i32_16x16x32_i8 per 16 x 16 tile of
+// tokens and weight rows and 32-block. What bounds it is issue: per (output,
+// 32-block) the order of the sums leaves one conversion (or subtraction, see below),
+// one or two products and one addition in f32, and a wave alone on its SIMD issues one
+// instruction per six cycles (two waves: three cycles; four: 2.4), while the MFMAs
+// add their own time. The kernels differ in how much of the machine a shape fills:
 //  * matmul_split_kernel, few tiles: the 128-blocks of one tile spread over 8
 //    waves, the terms handed over in LDS and added in order;
-//  * matmul_kernel<16 or 32 tokens>: a wave runs whole sums of 16 rows.
-// Measured (us per call, 8 weights in turn; before: one 64- or 32-token kernel
-// with one 128-block per barrier): n x k at 16 / 33 / 128 / 512 tokens
-//   1024 x 2560:  5.1 /  5.3 /  7.0 / 10.8   (before 24.3 / 14.2 / 14.2 / 14.3)
-//   4096 x 2560:  5.4 /  9.5 / 11.4 / 26.2   (       24.5 / 14.4 / 14.6 / 26.5)
-//   2560 x 4096:  6.1 /  8.7 / 15.9 / 29.4   (       37.3 / 24.0 / 24.5 / 31.0)
-//   2560 x 9728: 11.2 / 17.0 / 32.3 / 64.2   (       84.4 / 49.0 / 49.6 / 69.3)
-//   9728 x 2560:  9.6 / 11.5 / 20.5 / 57.4   (       24.7 / 16.0 / 21.7 / 56.9)
+//  * matmul_kernel<16 or 32 tokens>: a wave runs whole sums of 16 rows, weight rows as
+//    A and tokens as B, so that a lane holds four consecutive rows of one token, the
+//    scale a_d * w_d from the matrix core and sumi without a conversion, two or four
+//    128-blocks staged ahead;
+//  * matmul_block_kernel<32 or 64 tokens>: tokens as A, one 128-block staged ahead: the
+//    least start-up, and with 64 tokens the most work per weight, on large grids.
+// Measured (us per call, 8 weights in turn; one 64- or 32-token block kernel alone in
+// parentheses): n x k at 16 / 33 / 128 / 512 tokens
+//   1024 x 2560:  4.9 /  5.0 /  6.4 / 10.5   (24.1 / 14.1 / 14.2 / 14.3)
+//   4096 x 2560:  5.0 /  8.8 / 10.5 / 24.8   (24.3 / 14.2 / 14.3 / 24.8)
+//   2560 x 4096:  5.8 /  8.0 / 15.1 / 29.0   (37.0 / 24.1 / 24.2 / 29.7)
+//   2560 x 9728: 10.7 / 15.6 / 31.7 / 63.1   (83.9 / 48.7 / 49.4 / 67.1)
+//   9728 x 2560:  8.9 / 10.7 / 20.2 / 51.6   (24.5 / 15.7 / 20.0 / 51.7)
 #include "bp_device.hpp"
 #include "bp_kernels.hpp"
 
@@ -385,9 +388,152 @@ __global__ __launch_bounds__(64 * kSpWaves) void matmul_split_kernel(MatmulArgs 
     }
 }
 
+constexpr int kRowStride = 136;   // bytes per token row of the staged qs (128 + 8)
+
+template <int kTok> struct BlockStage {   // LDS image of one 128-block of the token tile
+    uint8_t qs[kTok * kRowStride];
+    float d[kTok * 4];   // [token][s]
+};
+
+// kTok tokens (A) x 64 weight rows (B) per workgroup, one 128-block a stage, scales
+// and conversions in f32. A wave owns 16 weight rows for all the tokens; a lane
+// holds four tokens of one row and reads their a_d of all four 32-blocks as 16-byte
+// LDS loads. Rows of the staged qs are padded to 136 bytes: the 16 rows that one
+// read touches start in different banks. Nothing past the last block is loaded.
+template <int kTok>
+__global__ __launch_bounds__(kMmThreads) void matmul_block_kernel(MatmulArgs a) {
+    constexpr int kTiles = kTok / 16;          // MFMA token tiles per wave
+    constexpr int kTpt = kMmThreads / kTok;    // staging threads per token
+    constexpr int kQpt = kTok / 32;            // 16-byte pieces per staging thread
+    __shared__ __attribute__((aligned(16))) BlockStage<kTok> st[2];
+    __shared__ uint2 lut[256];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const uint32_t nb1 = a.k / 128, nb8 = a.k / 32;
+    const uint32_t n0 = blockIdx.x * kMmRows, m0 = blockIdx.y * kTok;
+    const uint32_t g = lane >> 4, c = lane & 15;
+
+    fill_sign_table(lut, t, kMmThreads);
+
+    // token tile loads: thread t -> token t / kTpt, kQpt 16-byte pieces at
+    // 16 kQpt (t % kTpt); threads with t % kTpt < 4 also load d of s = t % kTpt
+    const uint32_t lt = t / kTpt, lq = t % kTpt;
+    const bool tok_ok = m0 + lt < a.m;
+    auto load_tok = [&](uint32_t b, uint4 (&q)[kQpt], float& dv) {
+#pragma unroll
+        for (int i = 0; i < kQpt; i++) q[i] = make_uint4(0u, 0u, 0u, 0u);
+        dv = 0.0f;
+        if (tok_ok && b < nb1) {
+            const uint8_t* src = a.acts + a.a_qs_offset + static_cast<uint64_t>(m0 + lt) * a.k + 128 * b + 16 * kQpt * lq;
+#pragma unroll
+            for (int i = 0; i < kQpt; i++) q[i] = *reinterpret_cast<const uint4*>(src + 16 * i);
+            if (lq < 4)
+                dv = *reinterpret_cast<const float*>(a.acts + a.a_d_offset +
+                                                     4 * (static_cast<uint64_t>(m0 + lt) * nb8 + 4 * b + lq));
+        }
+    };
+    auto store_tok = [&](int buf, const uint4 (&q)[kQpt], float dv) {
+        uint8_t* dst = st[buf].qs + lt * kRowStride + 16 * kQpt * lq;
+#pragma unroll
+        for (int i = 0; i < kQpt; i++) {
+            *reinterpret_cast<uint2*>(dst + 16 * i) = make_uint2(q[i].x, q[i].y);   // 8-byte aligned rows
+            *reinterpret_cast<uint2*>(dst + 16 * i + 8) = make_uint2(q[i].z, q[i].w);
+        }
+        if (lq < 4) st[buf].d[lt * 4 + lq] = dv;
+    };
+    // this lane's weight row (B column c of the wave's 16)
+    const uint32_t wn = n0 + 16 * wave + c;
+    const bool w_ok = wn < a.n;
+    auto load_w = [&](uint32_t b, uint4& q, uint16_t& d) {
+        q = make_uint4(0u, 0u, 0u, 0u);
+        d = 0;
+        if (w_ok && b < nb1) {
+            const uint64_t rb = static_cast<uint64_t>(wn) * nb1 + b;
+            q = *reinterpret_cast<const uint4*>(a.weights + a.w_qs_offset + 16 * rb);
+            d = *reinterpret_cast<const uint16_t*>(a.weights + a.w_d_offset + 2 * rb);
+        }
+    };
+
+    uint4 tq[kQpt], wq;
+    float tdv;
+    uint16_t wd16;
+    load_tok(0, tq, tdv);
+    load_w(0, wq, wd16);
+    store_tok(0, tq, tdv);
+    __syncthreads();
+
+    float acc[kTiles][4] = {};   // [token tile][j]: token 16 i + 4g + j, weight row wn
+    for (uint32_t b = 0; b < nb1; b++) {
+        const int cur = b & 1;
+        // next 128-block in flight
+        uint4 nq[kQpt], nwq;
+        float ndv;
+        uint16_t nwd;
+        load_tok(b + 1, nq, ndv);
+        load_w(b + 1, nwq, nwd);
+
+        const float wd = h2f(wd16);
+        const uint32_t wbits[4] = {wq.x, wq.y, wq.z, wq.w};
+        long bv[4];   // B for the four 32-blocks: elements 32 s + 8 g .. + 7 of the row, as +-1 bytes
+#pragma unroll
+        for (int s4 = 0; s4 < 4; s4++) {
+            const uint2 bw = lut[(wbits[s4] >> (8 * g)) & 0xFFu];
+            bv[s4] = static_cast<long>((static_cast<uint64_t>(bw.y) << 32) | bw.x);
+        }
+#pragma unroll
+        for (int i = 0; i < kTiles; i++) {
+            // a_d of this lane's 4 tokens, all four 32-blocks at once
+            float4 ad[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) ad[j] = *reinterpret_cast<const float4*>(&st[cur].d[(16 * i + 4 * g + j) * 4]);
+#pragma unroll
+            for (int s4 = 0; s4 < 4; s4++) {
+                // A: tokens 16 i + c, the same 8 elements
+                const uint2 av2 = *reinterpret_cast<const uint2*>(st[cur].qs + (16 * i + c) * kRowStride + 32 * s4 + 8 * g);
+                const long av = static_cast<long>((static_cast<uint64_t>(av2.y) << 32) | av2.x);
+                const i4v z = {0, 0, 0, 0};
+                const i4v sumi = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, bv[s4], z, 0, 0, 0);
+                // D[token 16 i + 4g + j][row c]; acc = acc + (a_d * w_d) * f32(sumi), blocks in order
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float adv = s4 == 0 ? ad[j].x : s4 == 1 ? ad[j].y : s4 == 2 ? ad[j].z : ad[j].w;
+                    const float scale = adv * wd;
+                    const float v = scale * static_cast<float>(sumi[j]);
+                    acc[i][j] = acc[i][j] + v;
+                }
+            }
+        }
+        store_tok(cur ^ 1, nq, ndv);
+        wq = nwq;
+        wd16 = nwd;
+        __syncthreads();
+    }
+
+    // output: y[out + token * n + row]
+    if (w_ok) {
+#pragma unroll
+        for (int i = 0; i < kTiles; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t tok = m0 + 16 * i + 4 * g + j;
+                if (tok < a.m) {
+                    uint16_t* y = a.y + a.out_offset + static_cast<uint64_t>(tok) * a.n + wn;
+                    if (a.accumulate) *y = f2h(h2f(*y) + acc[i][j]);
+                    else *y = f2h(acc[i][j]);
+                }
+            }
+    }
+}
+
 template <int kTok, int kStep>
 void launch_tiles(const MatmulArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((matmul_kernel<kTok, kStep>), dim3((a.n + kMmRows - 1) / kMmRows, (a.m + kTok - 1) / kTok),
+                       dim3(kMmThreads), 0, s, a);
+}
+
+template <int kTok>
+void launch_blocks(const MatmulArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL(matmul_block_kernel<kTok>, dim3((a.n + kMmRows - 1) / kMmRows, (a.m + kTok - 1) / kTok),
                        dim3(kMmThreads), 0, s, a);
 }
 
@@ -399,21 +545,41 @@ hipError_t launch_quantize_act_q8_0(const QuantArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// By how many workgroups a shape gives, against three per CU:
-//  * 16 x 16 tiles up to that: the split kernel (768 tiles: 4096 x 2560 at 33
-//    tokens 9.6 us, whole sums 9.5; 480 tiles, 2560 x 4096 at 33: 8.7, 13.1);
-//  * else 16 tokens a workgroup while that many fit (640: 2560 x 4096 at 256
-//    tokens 20.3 us, with 32 tokens 23.1; 1024: 4096 x 2560 at 256 17.2, 16.0);
-//  * else 32 tokens, four blocks a stage while its LDS holds all workgroups (640:
-//    2560 x 4096 at 512 29.4 us, two blocks 31.2), two beyond (1024: 4096 x 2560
-//    at 512 26.2, four blocks 30.2).
+// By how many workgroups a shape gives and by its 128-blocks; us per call, weights
+// of 8 tensors in turn, at n x k and tokens:
+//  * 64 tokens a workgroup where that still gives three per CU: with the most sums per
+//    staged weight (16384 x 2560 at 512 77.5, 32 tokens in two-block stages 86.9) and
+//    the least start-up (16384 x 128 at 512 10.2 and 20.5). Not where its last tile is
+//    padding for more than the 1/8 (at long k 1/16) that it gains (16384 x 9728 at 200
+//    156 and 140), nor past 80 blocks (6144 x 12288 at 512 161 and 155);
+//  * 16 x 16 tiles split by blocks up to three per CU (4096 x 2560 at 33: 768 tiles 9.6,
+//    whole sums 9.5; 2560 x 4096 at 33: 480, 8.7 and 13.1), fewer where the 8 waves
+//    have less than two blocks each (2560 x 640 at 64: 640 tiles, 5.5 and 4.7) or hardly
+//    one (512 tiles, 256 x 128 at 512: 3.8 and 3.5);
+//  * else 16 tokens while those workgroups fit three per CU (2560 x 4096 at 256 20.3,
+//    with 32 tokens 23.1); a single block has nothing to stage ahead (9728 x 128 at 64
+//    4.4, one-block stages 3.8);
+//  * else 32 tokens. Four-block stages while their LDS holds all workgroups (2560 x 4096
+//    at 512 29.4, two-block 31.2), two beyond (4096 x 2560 at 512 26.2, four-block
+//    30.2); one where the stages are few (3072 x 640 at 512 7.5, four-block 9.6; 6144 x
+//    1280 at 448 19.9, two-block 23.1), but, from two workgroups per CU, not with rows
+//    of a multiple of 1024 (2048 past three) elements, whose weight loads, a row per
+//    lane, then meet in few cache sets (4096 x 1024: 8.3 and 8.6 at 256 tokens, 10.5
+//    and 10.0 at 384; 2560 x 4096 at 1000 65.3, two-block 51.8).
 hipError_t launch_matmul_q1_0_q8_0(const MatmulArgs& a, hipStream_t s) {
-    const uint64_t three = 3ull * a.cu_count;
-    const uint64_t t16 = (a.m + 15) / 16, t32 = (a.m + 31) / 32, nx = (a.n + kMmRows - 1) / kMmRows;
-    if ((a.n + 15) / 16 * t16 <= three)
+    const uint64_t cus = a.cu_count, three = 3 * cus;
+    const uint64_t t16 = (a.m + 15) / 16, t32 = (a.m + 31) / 32, t64 = (a.m + 63) / 64;
+    const uint64_t nx = (a.n + kMmRows - 1) / kMmRows, tiles = (a.n + 15) / 16 * t16;
+    const uint32_t nb = a.k / 128;
+    const uint64_t pad = 64 * t64 * 24, full = 32 * t32;   // padded tokens, in 24ths of the 32-token tiles'
+    if (nx * t64 >= three && nb <= 80 && pad <= full * (nb <= 6 ? 32 : nb <= 20 ? 27 : 25))
+        launch_blocks<64>(a, s);
+    else if (tiles <= cus * (nb <= 2 ? 1 : nb < 16 ? 2 : 3))
         hipLaunchKernelGGL(matmul_split_kernel, dim3((a.n + 15) / 16, t16), dim3(64 * kSpWaves), 0, s, a);
-    else if (nx * t16 <= three)
+    else if (nx * t16 <= three && nb > 1)
         launch_tiles<16, 4>(a, s);
+    else if (nx * t32 <= three ? nb <= 12 && (nb % 8 != 0 || nx * t32 <= 2 * cus) : nb <= 20 && nb % 16 != 0)
+        launch_blocks<32>(a, s);
     else if (nx * t32 <= three)
         launch_tiles<32, 4>(a, s);
     else

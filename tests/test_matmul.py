@@ -217,13 +217,16 @@ def test_matmul_bit_exact(cuda, m, n, k, acc):
 
 # Every kernel choice at its edges (3 workgroups per CU of 256): the split kernel
 # (8 blocks a chunk: 1, 7, 8, 9 and 17 blocks), 16 tokens a workgroup (4 blocks a
-# stage), 32 tokens with 4 and with 2 blocks a stage; ragged rows and tokens, n not
-# a multiple of 4, offsets that are multiples of 4 only.
+# stage), 32 tokens with 1, with 4 (8 and 13 blocks) and with 2 blocks a stage (16 and
+# 21), 64 tokens with 1; ragged rows and tokens, n not a multiple of 4, offsets that
+# are multiples of 4 only.
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k,acc,shift", [
     (1, 1, 128, 0, 0), (17, 33, 7 * 128, 1, 4), (16, 16, 8 * 128, 0, 8), (33, 50, 9 * 128, 1, 0), (15, 70, 17 * 128, 0, 4),
     (193, 1000, 5 * 128, 1, 4), (200, 1001, 3 * 128, 0, 0), (250, 3001, 4 * 128, 0, 0), (250, 3004, 6 * 128, 1, 4),
-    (209, 5003, 6 * 128, 1, 4), (223, 7001, 3 * 128, 0, 4), (200, 8200, 2 * 128, 1, 0), (225, 6404, 5 * 128, 0, 8)])
+    (209, 5003, 6 * 128, 1, 4), (223, 7001, 3 * 128, 0, 4), (200, 8200, 2 * 128, 1, 0), (225, 6404, 5 * 128, 0, 8),
+    (20, 4100, 128, 1, 4), (209, 5003, 8 * 128, 1, 4), (209, 5004, 13 * 128, 0, 0), (225, 8001, 16 * 128, 0, 0),
+    (225, 6404, 21 * 128, 1, 8), (65, 24577, 128, 0, 8), (250, 12300, 3 * 128, 1, 4), (250, 12301, 7 * 128, 0, 0)])
 def test_matmul_kernel_choices_bit_exact(cuda, m, n, k, acc, shift):
     _say(f"[matmul choices] m={m} n={n} k={k} acc={acc} shift={shift}")
     rng = np.random.default_rng(m + n + k + shift)
