@@ -304,9 +304,11 @@ hipError_t launch_matvec_q1_0(const MatvecArgs& args, int mode, hipStream_t s) {
         // either way) 8.19 and 8.24. 16 waves where staging takes more than 12
         // (2560 x 9728: 8 waves 6.79; 2048 x 6144: 16 waves 4.87).
         // Below k = 3072 the staging is cheap and 16 blocks fill badly: 16 rows there
-        // (1024 x 2048 3.07, 4096 x 1024 2.87, tiles of 2 rows 3.20 and 3.18).
-        if (nb < 24) return launch(matvec_q1_0_kernel<1, 8, 1>, 16, std::min(2 * div_up(nb, 4), 16u));
-        const uint32_t rows = 2 * div_up(a.n_total, 2ull * cus * div_up(a.n_total, 32ull * cus));
+        // (1024 x 2048 3.07, 4096 x 1024 2.87, tiles of 2 rows 3.20 and 3.18). Nor do
+        // they help where 16 rows come out anyway: two tiles of 8 rows use each x read
+        // from LDS for more rows (4096 x 6144 5.79, tiles of 2 rows 6.00).
+        const uint32_t rows = nb < 24 ? 16 : 2 * div_up(a.n_total, 2ull * cus * div_up(a.n_total, 32ull * cus));
+        if (rows == 16) return launch(matvec_q1_0_kernel<1, 8, 1>, rows, std::min(2 * div_up(nb, 4), 16u));
         return launch(matvec_q1_0_kernel<1, 2, 1>, rows, a.k > 6144 ? 16 : 8);
     }
     if (mode == 0 && nb >= 32 && nb % 8 == 0 && a.n_total <= 24 * cus) {
@@ -323,22 +325,37 @@ hipError_t launch_matvec_q1_0(const MatvecArgs& args, int mode, hipStream_t s) {
     // and the terms fit 64 KB of LDS. By 16 / 32 / 64 rows: 12288 x 2048 4.68 /
     // 5.11 / 5.04 (8 rows 5.18), 19456 x 2560 6.9 / 6.9 / 7.2, 16384 x 2560 5.94 /
     // 5.68 / 5.51, 24576 x 4096 9.95 / 9.31 / 10.3, 151936 x 2560 37 / 27.5 / 26.8.
-    // Waves are a multiple of the CU's 4 SIMDs (with one tile row's 5 at k = 2560
-    // the first SIMD gets two waves of every workgroup); the normed sum of squares
-    // is defined over 256 threads (4 waves at least).
+    // 8 rows still where a plain x of up to 32 blocks is staged and that cost is no
+    // higher (9728 x 2560 4.93, 16 rows 5.19; with 33 blocks 6.71 and 6.79, with 40
+    // 7.09 and 6.86, and the normed staging costs more: 5.55 and 5.29); a few of these
+    // small workgroups (1/16 per CU) run beside the others (6160 x 2560 4.23, 32 rows
+    // 4.40; from 6400 the two are equal).
     const uint32_t tcols = (nb + 3) / 4;
     uint32_t rows = 8;
     if (a.n_total > 24 * cus) {
         const bool one_range = a.range[0].n == a.n_total;
         uint64_t best = ~0ull;
+        if (mode == 0 && tcols <= 8) best = 12ull * div_up(div_up(a.n_total, 8) - cus / 16, cus);
         for (uint32_t r : {16u, 32u, 64u}) {
             if (r > 16 && ((!one_range && (a.range[0].n % r || a.range[1].n % r)) || lds_bytes(r) > 65536)) continue;
             const uint64_t cost = static_cast<uint64_t>(div_up(a.n_total, static_cast<uint64_t>(r) * cus)) * (r + 4);
-            if (cost <= best) best = cost, rows = r;
+            if (cost < best || (cost == best && rows > 8)) best = cost, rows = r;
         }
     }
-    if (rows <= 16) {
-        const uint32_t waves = rows == 16 ? 4u : std::max(std::min(tcols, 16u), mode == 2 ? 4u : 1u);
+    // Waves. 8 rows: one tile each (with k = 2560's 5 on 4 SIMDs every workgroup adds
+    // to the first one, yet 8 waves of which 3 only stage took 5.34 at 9728 x 2560),
+    // but 8 where there are two or more workgroups of 10 to 16 per CU (6144 x 8192
+    // normed 7.14, 16 waves 8.78). 16 rows: 8 waves (12288 x 4224 6.84, 4 waves 7.11;
+    // 19456 x 16384 23.9 and 27.6), 4 where x is small (under 20 blocks both the same)
+    // or the normed sum, over 256 threads (4 waves at least), holds the others up
+    // (9728 x 4096 6.37, 8 waves 6.45; past k = 8192 again 8).
+    if (rows == 8) {
+        const bool two = a.n_total > 16 * cus && tcols >= 10;
+        const uint32_t waves = two ? 8u : std::max(std::min(tcols, 16u), mode == 2 ? 4u : 1u);
+        return mode == 0 ? launch(matvec_q1_0_kernel<0, 8, 1>, rows, waves) : launch(matvec_q1_0_kernel<2, 8, 1>, rows, waves);
+    }
+    if (rows == 16) {
+        const uint32_t waves = (mode == 0 && nb >= 20) || a.k > 8192 ? 8u : 4u;
         return mode == 0 ? launch(matvec_q1_0_kernel<0, 8, 1>, rows, waves) : launch(matvec_q1_0_kernel<2, 8, 1>, rows, waves);
     }
     // Two rows per lane (x read from LDS once for both, two independent chains:

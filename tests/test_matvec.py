@@ -446,8 +446,8 @@ def test_matvec_rejects_bad_shapes(cuda, monkeypatch):
                                             [(0, 0, 24, 0)])
 
 
-# The f16-order kernel's larger grids (32 or 64 rows a workgroup, 8 waves; 16 rows
-# where a range is no multiple of 32), with rows past the last whole workgroup.
+# The f16-order kernel's largest grids (32 or 64 rows a workgroup; 16 rows where a
+# range is no multiple of 32), with rows past the last whole workgroup.
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,k,acc", [(65600, 128, 0), (65601, 512, 1), (131072, 128, 0), (131072 + 33, 256, 1)])
 def test_matvec_large_grids(cuda, monkeypatch, n, k, acc):
@@ -467,7 +467,7 @@ def test_matvec_large_grids(cuda, monkeypatch, n, k, acc):
 @pytest.mark.gpu
 @pytest.mark.parametrize("sizes", [(32768, 32800), (32784, 32784), (16, 32768, 32784), (64, 131072), (0, 65568)])
 def test_matvec_fused_normed_large_grids(cuda, monkeypatch, sizes):
-    """Each range must be the product one range alone gives (small grids, bit-exact above)."""
+    """Each range must be the product that 1024 of its rows alone give (small grids, bit-exact above)."""
     import torch
     k = 256
     _say(f"[matvec normed large] sizes={sizes}")
@@ -483,37 +483,41 @@ def test_matvec_fused_normed_large_grids(cuda, monkeypatch, sizes):
     got_d, want_d = _dev(act), _dev(act)
     m.dispatch_matvec_q1_0_fused_normed(w_d.data_ptr(), got_d.data_ptr(), n_d.data_ptr(), k, 0, 0, ranges)
     for d, q, n, o in ranges:
-        for lo in range(0, n, 8192):   # pieces that run one tile per wave
-            c = min(8192, n - lo)
+        for lo in range(0, n, 1024):   # 8 rows a workgroup, one tile a wave
+            c = min(1024, n - lo)
             m.dispatch_matvec_q1_0_fused_normed(w_d.data_ptr(), want_d.data_ptr(), n_d.data_ptr(), k, 0, 0,
                                                 [(d + 2 * lo * (k // 128), q + 16 * lo * (k // 128), c, o + lo)])
     torch.cuda.synchronize()
     assert torch.equal(got_d, want_d)
 
 
-# The f16-order kernel's plan at its edges: 16 rows (from 24 rows per CU on), 32
-# with one and two rows per lane, 64; long rows in tiles of 4 rows; rows past the
-# last whole workgroup, blocks past the last whole tile.
+# The f16-order kernel's plan at its edges: 8 rows up to 24 per CU and a few more,
+# and between 32 and 40 per CU (up to 32 blocks), with 8 waves for several tiles each;
+# 16 rows with 4 and 8 waves, 32 with one and two rows per lane, 64; long rows in
+# tiles of 4 rows; rows past the last whole workgroup, blocks past the last whole tile.
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,k,acc", [(6144, 1152, 0), (6145, 1152, 1), (8192 - 3, 2048, 0), (8192, 2560, 1), (11000, 640, 0),
                                      (16384, 1024, 0), (16389, 2048, 1), (1, 4096, 0), (1027, 4096, 1), (2560, 4096, 1),
-                                     (3000, 5120, 0), (2050, 4224, 0), (514, 16384, 0)])
+                                     (3000, 5120, 0), (2050, 4224, 0), (514, 16384, 0), (6272, 1024, 0), (6273, 1024, 1),
+                                     (8193, 3072, 0), (10243, 4096, 1), (10241, 2560, 0), (5001, 5248, 1), (4097, 8320, 0),
+                                     (9001, 4224, 0), (12289, 8320, 1)])
 def test_matvec_plan_choices(cuda, monkeypatch, n, k, acc):
     test_matvec_large_grids(cuda, monkeypatch, n, k, acc)
 
 
 # The silu matvec in tiles of 2 rows x 16 blocks: from 2 rows per workgroup to 32
-# and a second round of workgroups, odd rows, 8 and 16 waves.
+# and a second round of workgroups, odd rows, 8 and 16 waves; 16 rows in tiles of 8.
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,k,acc", [(1, 3072, 0), (513, 3072, 1), (1024, 3072, 0), (1025, 3200, 1), (2560, 2944, 0),
-                                     (300, 6144, 0), (301, 6272, 1), (100, 16384, 0), (8192, 3072, 0), (8193, 3072, 1)])
+                                     (300, 6144, 0), (301, 6272, 1), (100, 16384, 0), (8192, 3072, 0), (8193, 3072, 1), (3585, 3072, 0),
+                                     (4095, 3200, 1), (4096, 6272, 0), (8190, 2944, 0)])
 def test_matvec_silu_plan_choices(cuda, monkeypatch, n, k, acc):
     test_matvec_silu(cuda, monkeypatch, "f16", n, k, acc)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("sizes,k", [((8192, 16384), 2048), ((8192 + 16, 16384), 2048), ((4096, 2048, 64), 1024), ((9728, 9728), 640),
-                                     ((16384,), 1152)])
+                                     ((16384,), 1152), ((5008,), 5248), ((4096, 1024, 1024), 6144), ((9728,), 8320)])
 def test_matvec_fused_normed_plan_choices(cuda, monkeypatch, sizes, k):
     """Each range must be the product that 1024 of its rows alone give (small grids, bit-exact above)."""
     _say(f"[matvec normed plan] sizes={sizes} k={k}")
