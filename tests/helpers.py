@@ -14,7 +14,7 @@ import numpy as np
 import oracle as orc
 from bonsai_pot_amd.layout import Config, kv_buffer_bytes, kv_layer_offsets
 
-TOL_MAX_ABS = 2e-3      # attention output vs f32-softmax oracle (north-star bar)
+TOL_MAX_ABS = 2e-3      # attention output vs f32-softmax oracle
 TOL_REL_L2 = 1e-3
 # (what, max_abs, rel_l2, max_ulp, n_off, n_big) of every attention comparison
 # in this process. Over the n_big outputs of magnitude >= ULP_MIN_MAG (where an
@@ -239,7 +239,7 @@ def write_outlier_rows(sc: Scenario, il: int, n_rows: int, seed: int, frac: floa
     """Oracle-written cache rows [0, n_rows) of layer il from an independent
     seeded K/V scenario, with `frac` of the rows' K scaled x8 before
     quantization (a w_k_norm of 8.0 for those rows, exact in f16) — the
-    softmax max-tracking stress of BASELINE configs[4]. Returns the rows."""
+    stress of the softmax max tracking. Returns the rows."""
     cfg = sc.cfg
     pre = Scenario(cfg, sc.max_seq, n_rows, seed=seed, with_q=False)
     pre.kv_k, pre.kv_v = sc.kv_k, sc.kv_v

@@ -3,7 +3,7 @@ only include/bonsai_pot_hip.h (and the HIP runtime API for its own device
 buffers) and links libbonsai_pot_hip.so, as the reference-side -sys crate
 would. CPU: the header is self-sufficient C99 and the program links against
 the library; without a device the program reports BP_ERR_NO_DEVICE through
-the ABI's own error strings. GPU: one decode step of configs[1]'s shape,
+the ABI's own error strings. GPU: one decode step of a Bonsai-4B layer at ctx 4096,
 both as the reference's three dispatches and as the fused entry point, run by
 the C program and compared with the oracle (cache bytes bit-exact, attention
 within the tolerance)."""

@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 
 from bonsai_pot_amd import layout
-from helpers import DeviceScenario, Scenario
+from helpers import DeviceScenario, Scenario, launches_of
 
 pytestmark = pytest.mark.gpu
 
@@ -92,14 +92,31 @@ def test_graph_decode_steps(cuda, monkeypatch, wide_min):
     _check_replays(dev, body, f"decode wide_min={wide_min}")
 
 
+@pytest.mark.parametrize("pos", [300, 100])
+def test_graph_decode_one_launch_steps(cuda, pos):
+    """Fused steps of two layers and the plain entry point in one launch each (8 waves a
+    KV head; the plain one on 101 rows: one split, which stores the output itself)."""
+    _say(f"[graph] decode steps in one launch pos={pos}")
+    sc = _scenario(1, pos, seed=5150 + pos)
+    dev = DeviceScenario(sc, upload_kv=True)
+
+    def body():
+        dev.decode_step(0, pos)
+        dev.decode_step(1, pos)
+        dev.decode(1, pos)
+    assert launches_of(dev.model, body) == 3
+    _check_replays(dev, body, f"decode one launch pos={pos}")
+
+
 @pytest.mark.parametrize("entry", ["step", "dispatch"])
-@pytest.mark.parametrize("m,pos", [(512, 0), (2048, 0), (64, 4096), (300, 64)])
+@pytest.mark.parametrize("m,pos", [(512, 0), (2048, 0), (64, 4096), (300, 64), (64, 1000)])
 def test_graph_prefill(cuda, m, pos, entry):
     """The fused prefill step (preparation pass + attention kernel) and the
     plain attention dispatch (image pass + attention kernel): the 16x16
     kernels (512 tokens), prefill32_kernel (2048), the key-split kernel and
-    its merge pass (64 tokens on 4096 rows), and a chunk that mixes cache rows
-    and new rows (300 on 64)."""
+    its merge pass (64 tokens on 4096 rows), a chunk that mixes cache rows
+    and new rows (300 on 64), and prefill32_kernel with its keys split (64 on
+    1000)."""
     _say(f"[graph] prefill {entry} m={m} pos={pos}")
     # the dispatch attends rows [0, pos + m): all of them written beforehand
     sc = _scenario(m, pos, seed=5200 + m + pos, rows=pos if entry == "step" else pos + m)

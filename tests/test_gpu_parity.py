@@ -132,7 +132,7 @@ def test_decode_long_context(cuda, pos):
 
 
 def test_decode_ctx32k_with_outlier_rows(cuda):
-    """Config 5: ctx 32768 (32769 rows), 1% of key rows x8 before quantization
+    """Decode at ctx 32768 (32769 rows), 1% of key rows x8 before quantization
     (x8 = a w_k_norm of 8.0 for those rows, exact in f16)."""
     _say("[decode] ctx32k outliers")
     cfg = layout.Config(n_layer=1)
@@ -204,7 +204,7 @@ def test_attention_non_causal_multi_token(cuda, m, pos):
 
 @pytest.mark.parametrize("m,pos_base", [(2048, 0), (2048, 2048), (64, 16384)])
 def test_prefill_full_size_sampled_rows(cuda, m, pos_base):
-    """pp2048 (metric), config 4 (2048-token chunk over a 2048-row cache) and
+    """2048 tokens from an empty cache and over a 2048-row cache, and
     the bench's chat-turn shape (64 tokens over 16384 rows: the key-split
     kernel at its default 32 splits): the whole output is computed on the
     GPU, the oracle checks sampled tokens spread over every 64-token tile,
@@ -343,11 +343,11 @@ def test_prefill_with_outlier_key_rows(cuda, monkeypatch, m, pos_base, hpw):
     assert_attn_close(dev.out_f32(), want, f"prefill outliers m={m} pos={pos_base} hpw={hpw}")
 
 
-def test_config1_real_cache_last_layer(cuda):
-    """configs[1]'s real cache: n_layer 36, ctx 4096, the fused step on the last
+def test_bonsai4b_real_cache_last_layer(cuda):
+    """Bonsai-4B's real cache: n_layer 36, ctx 4096, the fused step on the last
     layer (35). Cache rows written by the oracle for layer 35 only; after the
     step layer 35 gains row 4096 and every other layer's bytes are untouched."""
-    _say("[config1] n_layer=36 ctx=4096 layer 35")
+    _say("[real cache] n_layer=36 ctx=4096 layer 35")
     cfg = layout.Config(n_layer=36)
     pos = 4096
     sc = Scenario(cfg, max_seq=pos + 64, m_tokens=1, seed=4135)
