@@ -1,6 +1,6 @@
 """Benchmark of the MI355X attention hot path (one JSON line on stdout).
 
-Headline workload (value): BASELINE configs[1] — Bonsai-4B decode attention
+Headline workload (value): Bonsai-4B decode attention
 over all 36 layers at ctx 4096, batch 1. One step = for each layer:
 q_norm_rope (1 token) -> kv_writeback of row 4096 -> split-K decode
 attention over 4097 rows, replayed from a HIP graph. Inputs are resident in
@@ -10,8 +10,8 @@ Cache, so every step streams the KV cache from HBM.
 value = algorithmic bytes per step / step time, with per layer
 4097 rows x 2304 B (K+V: 2 x (128 qs + 4 x 4 B d)) + 16384 B (q in, out).
 
-Also reported: decode at ctx 32768 (config 5, rotating over 8 layers),
-prefill pp2048 (metric) and the 2048-on-2048 chunked prefill (config 4) in
+Also reported: decode at ctx 32768 (rotating over 8 layers),
+prefill pp2048 and the 2048-on-2048 chunked prefill in
 TFLOP/s of unmasked QK^T + PV work, the Bonsai-4B per-layer Q1_0 decode
 matvecs (fused normed q/k/v, o, fused normed gate/up, silu down) over 36
 layers of distinct weights in GB/s, the prefill projections (Q8_0
@@ -703,7 +703,7 @@ def main():
         "vs_baseline": None,
         "dtype": "f32 (i8 Q8_0 cache, f16 q/out)",
         "data": "synthetic (seeded N(0,1) q/k/v through kv_writeback; no model weights)",
-        "config": {"workload": "configs[1]: Bonsai-4B decode attention, 36 layers, ctx 4096, batch 1 "
+        "config": {"workload": "Bonsai-4B decode attention, 36 layers, ctx 4096, batch 1 "
                                "(fused q_norm_rope + kv_writeback + split-K decode per layer, HIP graph)",
                    "n_head": 32, "n_kv_head": 8, "head_dim": 128, "ctx": 4096, "layers": 36,
                    "parallelism": "none (1 GPU)"},

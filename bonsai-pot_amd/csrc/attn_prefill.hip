@@ -13,11 +13,11 @@
 //    two waves of each SIMD one phase apart (its own comment below). Grids
 //    that leave CUs idle take one tile per workgroup instead of two and, on
 //    few tiles, split the keys as well (then prefill_merge_kernel).
-// 2. Image pass + prefill_kernel<1, 4> (few key chunks; <1, 8> when forced):
-//    one query head per wave on v_mfma_f32_16x16x32_f16, four (two) workgroups
+// 2. Image pass + prefill_kernel<1, 4> (few key chunks; <1, 8> where 4 waves a
+//    workgroup do not fit the CUs and the chunks are fewest): one query head per wave on v_mfma_f32_16x16x32_f16, four (two) workgroups
 //    per (KV head, tile pair), so that small grids still fill the CUs.
 // 3. prefill_split_kernel + prefill_merge_kernel (few tokens over a long
-//    cache): the keys split over workgroups that read the cache's Q8_0 rows
+//    cache, or an output across q): the keys split over workgroups that read the cache's Q8_0 rows
 //    themselves (no image), partials merged by their log-sum-exp weights.
 //
 // prefill_kernel, a flash-attention over LDS tiles of the image:
@@ -948,10 +948,7 @@ __device__ __forceinline__ f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) {
 __device__ __forceinline__ f32x16 mfma32_resid(i32x8 a, i32x8 b, f32x16 c, int sa, int sb) {
     return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 2, 2, 0, sa, 0, sb);
 }
-// Workgroup barriers without a memory fence (a workgroup-scope fence would
-// also wait for the copies still in flight). Before the first, this wave's
-// LDS reads are complete; before the second, also its copies into LDS.
-__device__ __forceinline__ void barrier_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// lds_barrier, and also this wave's copies into LDS complete.
 __device__ __forceinline__ void barrier_copies() {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
@@ -1275,7 +1272,7 @@ __global__ __launch_bounds__(512) void prefill32_kernel(PrefillArgs a) {
                 have_p = false;
             }
             if (live) qk(par ? kst1 : kst0);
-            barrier_lds();
+            lds_barrier();
             // K(i+1) and V(i) are copied during the VALU phase (their issue
             // would delay the MFMAs; here the other wave's MFMA phase covers
             // it): 10 copies of 1 KB, two at each softmax hook.
@@ -1329,7 +1326,7 @@ __global__ __launch_bounds__(512) void prefill32_kernel(PrefillArgs a) {
                 xml[64 + lane] = l_tot;
             }
         }
-        barrier_lds();
+        lds_barrier();
         if (!is_x) {
             const float mx = xml[c], lx = xml[64 + c];
             const float mm = fmaxf(m_run, mx);
@@ -1342,7 +1339,7 @@ __global__ __launch_bounds__(512) void prefill32_kernel(PrefillArgs a) {
             if (a.n_ksplit > 1) write_partial(mm, l_tot * ey + lx * ex);
             else write_out(l_tot * ey + lx * ex);
         }
-        barrier_lds();   // the merge area is the next tile's stages
+        lds_barrier();   // the merge area is the next tile's stages
     };
 
     const uint32_t tile_b = a.n_tiles - 1 - pair, tile_a = a.tiles_per_wg == 1 ? tile_b : pair;   // tile_b >= tile_a

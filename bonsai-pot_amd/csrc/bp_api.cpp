@@ -302,7 +302,7 @@ bp_status bp_model_create(const bp_config* cfg, uint32_t max_seq, int device, bp
     // choices equal the reference's. Opt-in "mfma": exact integer sums of x
     // rounded to 15 bits per block on the i8 matrix cores (closer to the
     // exact product, not the reference's bits); "auto": f16 below the
-    // streaming size, MFMA from it on (the LM head, 2.2x faster there).
+    // streaming size, MFMA from it on (the LM head: 151936 x 2560 25.8 us, 20.6).
     m->matvec_arith = 1;
     if (const char* env = std::getenv("BP_MATVEC_ARITH")) {
         if (std::strcmp(env, "auto") == 0) m->matvec_arith = 0;

@@ -100,4 +100,8 @@ __device__ __forceinline__ float i8f(uint32_t w, int i) {
     return static_cast<float>(static_cast<int32_t>(w << (24 - 8 * i)) >> 24);
 }
 
+// Workgroup barrier without a memory fence (a workgroup-scope fence would also wait
+// for global loads and copies still in flight): this wave's LDS accesses are complete.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 }  // namespace bp

@@ -92,9 +92,10 @@ struct PrefillArgs {
     uint32_t pos;             // first query's RoPE/cache position when causal
     uint32_t causal;          // 1: token m sees rows [0, pos+m]; 0: rows [0, pos)
     uint32_t n_tiles;         // ceil(m_tokens / kPrefillTileTok)
-    uint32_t heads_per_wave;  // 2: prefill32_kernel (4 heads x 32 tokens per role); 1: prefill_kernel (two or four workgroups per tile pair)
+    uint32_t heads_per_wave;  // 2: prefill32_kernel (4 heads x 32 tokens per role); 1: prefill_kernel (two or four
+                              // workgroups per tile pair), or with direct prefill_split_kernel
     uint32_t tiles_per_wg;    // prefill32_kernel: 2 (a zig-zag pair of tiles) or 1
-    uint32_t wg_waves;        // with 1 head per wave: 8 (two head sets) or 4 (four, one head each)
+    uint32_t wg_waves;        // prefill_kernel: 8 (two head sets) or 4 (four, one head each)
     // Key split: n_ksplit > 1 workgroups of prefill_split_kernel (direct = 1) per
     // (KV head, tile pair), or of prefill32_kernel (tiles_per_wg = 1) per (KV
     // head, tile), each over split_chunks 64-row chunks of the key range, write

@@ -113,9 +113,6 @@ __device__ __forceinline__ void fill_sign_table(uint2* lut, uint32_t t, uint32_t
     }
 }
 
-// All LDS accesses of the workgroup's waves done; global loads stay in flight.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // y[out + tok * n + row + r] for four rows; vec: 8-byte aligned and n a multiple of 4.
 __device__ __forceinline__ void store4(uint16_t* y, uint32_t row, uint32_t n, bool vec, uint32_t accumulate, const float* v) {
     if (vec) {

@@ -184,9 +184,9 @@ bp_status bp_dispatch_attention_prefill_step(bp_model* model, void* act, const v
  * offsets are f16-element offsets into `act` and must be multiples of 8.
  * y[out_off + r] = f16(sum_b d[r][b] * sum_e (+-x[e])) (or, with accumulate,
  * f16(f32(y) + that)). Arithmetic (environment BP_MATVEC_ARITH at
- * bp_model_create): "f16" = the reference's f16 block sums, bit for bit;
+ * bp_model_create): default "f16" = the reference's f16 block sums, bit for bit;
  * "mfma" = exact integer sums of x rounded to 15 bits of each block's max |x|,
- * f32 scaling; default "auto" = f16 below 32768 rows, mfma from there on. */
+ * f32 scaling; "auto" = f16 below 32768 rows, mfma from there on. */
 bp_status bp_dispatch_matvec_q1_0(bp_model* model, const void* weights, void* act, uint32_t k,
                                   uint32_t n, uint32_t w_d, uint32_t w_qs, uint32_t in_off,
                                   uint32_t out_off, uint32_t accumulate);
