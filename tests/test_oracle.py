@@ -97,7 +97,7 @@ def test_snapshot_offsets_no_overlap():
 
 
 def test_kv_layout_u32_range_at_36x32768():
-    # SURVEY-derived: qs base 150,994,944 B; whole buffer 1,358,954,496 B < 2^32.
+    # qs base 150,994,944 B; whole buffer 1,358,954,496 B < 2^32.
     d, q = orc.kv_layer_offsets(36, 1024, 32768, 0)
     assert (d, q) == (0, 150_994_944)
     assert orc.kv_buffer_bytes(36, 1024, 32768) == 1_358_954_496 < 2**32
