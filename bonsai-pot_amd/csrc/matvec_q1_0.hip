@@ -314,7 +314,9 @@ hipError_t launch_matvec_q1_0(const MatvecArgs& args, int mode, hipStream_t s) {
     if (mode == 0 && nb >= 32 && nb % 8 == 0 && a.n_total <= 24 * cus) {
         // Long rows, few of them: one workgroup per CU here too, tiles of 4 rows
         // (2560 x 4096 4.23 -> 3.97, 4096 x 4096 4.40 -> 4.31, 1024 x 4096 3.24 ->
-        // 3.14; with k = 2048 the smaller workgroups below are as fast).
+        // 3.14; with k = 2048 the smaller workgroups below are as fast). Whole tiles of 8
+        // blocks only: past one the gain is gone on most sizes (k = 4224: 1024 / 2560 /
+        // 4096 / 6144 rows 3.8 / 4.3 / 4.5 / 5.4, below 3.7 / 4.5 / 4.6 / 5.2).
         const uint32_t rows = 4 * div_up(a.n_total, 4 * cus), tiles = rows / 4 * (nb / 8);
         return launch(matvec_q1_0_kernel<0, 4, 1>, rows, std::min(tiles, 16u));
     }
